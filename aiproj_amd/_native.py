@@ -20,6 +20,7 @@ LIBRARY_PATH = Path(__file__).resolve().parent / "libkvfp8.so"
 
 # enum kvfp8_dtype in include/kvfp8.h
 F32, F16, BF16, E4M3FN, I32, I64 = 0, 1, 2, 3, 4, 5
+ELIMIT = -6        # KVFP8_ELIMIT: a size beyond what the kernels support
 
 TORCH_TO_CODE = {
     torch.float32: F32,
@@ -56,6 +57,9 @@ SIGNATURES = {
     "kvfp8_silu_mul": (_INT, [_P, _INT, _I64, _I32, _I64, _P, _I64, _P]),
     "kvfp8_prefill_attention": (_INT, [_P, _P, _P, _INT, _I64, _I32, _I32, _I32, _P, _INT, _I32, _I32,
                                        ctypes.c_float, _P, _P, _P]),
+    "kvfp8_prefill_backward_workspace_bytes": (_I64, [_INT, _I64, _I32, _I32, _I32, _I32, _I32, _INT]),
+    "kvfp8_prefill_attention_backward": (_INT, [_P, _P, _P, _P, _P, _P, _INT, _I64, _I32, _I32, _I32, _P, _INT, _I32,
+                                                _I32, ctypes.c_float, _P, _P, _P, _P, _I64, _P]),
     "kvfp8_timing_enable": (_INT, [_I32]),
     "kvfp8_timing_read": (_INT, [ctypes.POINTER(ctypes.c_double), ctypes.POINTER(_I64)]),
     "kvfp8_strerror": (ctypes.c_char_p, [_INT]),

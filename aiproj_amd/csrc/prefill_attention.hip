@@ -27,18 +27,13 @@
 //                           from a 16-bit v_perm transpose of eight V rows
 // bf16 inputs run bf16 products, f16 inputs f16 products, float32 inputs a bf16
 // hi + lo split of every operand (three products each, about 16 mantissa bits).
-#include "kvfp8_common.h"
+#include "mfma_tiles.h"
 
 #include <type_traits>
 
 namespace kvfp8 {
 
 namespace {
-
-typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
-typedef float f32x4_t __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 
 constexpr int kPThreads = 256;     // 4 waves
 constexpr int kKeys = 64;          // keys per KV block
@@ -72,16 +67,6 @@ struct Opnd {
     u32x4_t l;
 };
 
-template <bool kF16>
-__device__ __forceinline__ f32x4_t mma16(u32x4_t a, u32x4_t b, f32x4_t c) {
-    if constexpr (kF16)
-        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, b),
-                                                     c, 0, 0, 0);
-    else
-        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a),
-                                                      __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
-}
-
 // c += a b, with the split inputs' hi hi + hi lo + lo hi terms.
 template <bool kF16, bool kSplit>
 __device__ __forceinline__ f32x4_t mma(const Opnd<kSplit>& a, const Opnd<kSplit>& b, f32x4_t c) {
@@ -102,19 +87,6 @@ __device__ __forceinline__ uint32_t bf16_bits(float x) {
 }
 __device__ __forceinline__ uint32_t f16_bits(float x) {
     return (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)x);
-}
-
-typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
-typedef float f32x2_t __attribute__((ext_vector_type(2)));
-
-// Two floats -> one dword of two 16-bit values, rounded to nearest even (one
-// v_cvt_pk_bf16_f32 / v_cvt_pk_f16_f32).
-template <bool kF16>
-__device__ __forceinline__ uint32_t pack2(float x0, float x1) {
-    const f32x2_t v = {x0, x1};
-    if constexpr (kF16) return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, f16x2_t));
-    else return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2_t));
 }
 
 // Maximum over lanes l, l ^ 16, l ^ 32 and l ^ 48. Each permlane swap leaves the
@@ -477,14 +449,6 @@ constexpr int kXcds = 8;           // workgroups are dispatched round-robin over
 constexpr int kGroupUnits = 8;     // units per longest-first group (their K/V: 8 x 512 KB at L 1024, D 128)
 constexpr int kFaBufs = 3;         // K/V block buffers in LDS
 
-// Wave-uniform loads through the scalar data cache: a pointer into the constant
-// address space (read-only for the kernel's lifetime) lets the compiler use
-// s_load. A plain load of this memory would be a vector load here (the kernel also
-// stores to global memory), and the compiler would then wait for every
-// vector-memory operation in flight, K/V prefetches included.
-typedef __attribute__((address_space(4))) const int64_t* const_i64_ptr;
-typedef __attribute__((address_space(4))) const int32_t* const_i32_ptr;
-
 // One work item: query block qb of a unit (sequence b, KV head hk, head block hb).
 struct FaItem {
     int32_t s0;        // first token of the sequence
@@ -523,17 +487,7 @@ __device__ __forceinline__ bool fa_item(const PrefillArgs& a, const FaSchedule& 
         const int32_t b = unit / (a.hkv * a.blocks_per_kv);
         const int32_t rest = unit - b * a.hkv * a.blocks_per_kv;
         int64_t s0, s1;
-        if (a.cu64) {
-            const const_i64_ptr cu = (const_i64_ptr)a.cu;
-            s0 = cu[b];
-            s1 = cu[b + 1];
-        } else {
-            const const_i32_ptr cu = (const_i32_ptr)a.cu;
-            s0 = cu[b];
-            s1 = cu[b + 1];
-        }
-        s0 = s0 < 0 ? 0 : s0;
-        s1 = s1 > a.total_tokens ? a.total_tokens : s1;
+        seq_bounds(a.cu, a.cu64, b, a.total_tokens, &s0, &s1);
         int64_t len64 = s1 > s0 ? s1 - s0 : 0;
         len64 = len64 < a.max_len ? len64 : a.max_len;
         const int L = (int)len64;

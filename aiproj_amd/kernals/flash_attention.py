@@ -14,9 +14,11 @@ Same interface as the reference:
 * `FlashAttentionFunction.apply(q, k, v, cum_seq, batch_max_seq_len)` (reference
   `:10-48`) with `scale = 1/sqrt(D)`.
 
-The backward (`flash_attention_backward`, reference `:213-...`) is training-side and not
-part of the prefill path: it is written with PyTorch float32 operations on the device
-from the saved `lse`, sequence by sequence (it reads the sequence bounds on the host).
+The backward (`flash_attention_backward`, reference `:213-...`) is one call of the HIP
+kernels behind `kvfp8_prefill_attention_backward` for head sizes up to 128: products of
+float32 accuracy on the matrix cores, no host synchronization. Other head sizes, mixed
+dtypes, strided inputs and CPU tensors take PyTorch float32 operations, sequence by
+sequence (that path reads the sequence bounds on the host).
 
 Head sizes 1 to 512 (`ValueError` otherwise), like the reference, which pads any size
 to a power of two (`:72`): multiples of 8 up to 128 run on the matrix-core kernels, every
@@ -61,8 +63,45 @@ def flash_attention_forward(q: t.Tensor, k: t.Tensor, v: t.Tensor, cum_seq: t.Te
     return output, lse
 
 
+_MAX_BACKWARD_HEAD = 128
+
+
+def _native_backward(q, k, v, output, lse, cum_seq, grad_output, batch_max_seq_len, scale):
+    """dq, dk, dv from the HIP kernels, or None for what they do not take."""
+    rows = (q, k, v, output, grad_output)
+    if (q.device.type != "cuda" or q.dtype not in _DTYPES or q.ndim != 3 or q.shape[2] > _MAX_BACKWARD_HEAD
+            or q.numel() == 0 or lse.dtype != t.float32 or cum_seq.dtype not in (t.int32, t.int64) or cum_seq.ndim != 1
+            or cum_seq.shape[0] < 2 or not 0 < int(batch_max_seq_len) < 2 ** 31):
+        return None
+    total, hq, d = q.shape
+    hkv = k.shape[1]
+    if (any(x.dtype != q.dtype or not x.is_contiguous() for x in rows) or k.shape != v.shape
+            or k.shape != (total, hkv, d) or hq % hkv or output.shape != q.shape or grad_output.shape != q.shape
+            or lse.shape != (total, hq) or not lse.is_contiguous() or not cum_seq.is_contiguous()
+            or any(x.device != q.device for x in (*rows, lse, cum_seq))):
+        return None
+    code = _native.dtype_code(q.dtype)
+    batch, longest = cum_seq.shape[0] - 1, int(batch_max_seq_len)
+    aligned = all(x.data_ptr() % 16 == 0 for x in (q, k, v, grad_output))
+    size = _native.lib().kvfp8_prefill_backward_workspace_bytes(code, total, hq, hkv, d, batch, longest, aligned)
+    dq, dk, dv = t.empty_like(q), t.empty_like(k), t.empty_like(v)
+    workspace = t.empty(size, dtype=t.uint8, device=q.device)
+    rc = _native.lib().kvfp8_prefill_attention_backward(
+        q.data_ptr(), k.data_ptr(), v.data_ptr(), output.data_ptr(), lse.data_ptr(), grad_output.data_ptr(), code,
+        total, hq, hkv, d, cum_seq.data_ptr(), _native.dtype_code(cum_seq.dtype), batch,
+        longest, float(scale), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), workspace.data_ptr(), size,
+        _native.stream_handle(q.device))
+    if rc == _native.ELIMIT:      # returned before anything is launched
+        return None
+    _native.check(rc, "kvfp8_prefill_attention_backward")
+    return dq, dk, dv
+
+
 def flash_attention_backward(q, k, v, output, lse, cum_seq, grad_output, batch_max_seq_len, scale):
-    """dq, dk, dv of the causal varlen attention (float32 math, per sequence)."""
+    """dq, dk, dv of the causal varlen attention (float32 products, rounded to the inputs' dtypes)."""
+    grads = _native_backward(q, k, v, output, lse, cum_seq, grad_output, batch_max_seq_len, scale)
+    if grads is not None:
+        return grads
     total, hq, d = q.shape
     hkv = k.shape[1]
     g = hq // hkv

@@ -237,6 +237,26 @@ int kvfp8_prefill_attention(const void* q_dev, const void* k_dev, const void* v_
                             float scale, void* out_dev, float* lse_dev, void* stream);
 
 /*
+ * Backward of kvfp8_prefill_attention: dq [T, Hq, D], dk and dv [T, Hkv, D] (the inputs'
+ * dtype) from q, k, v, the forward's out and lse, and grad_out [T, Hq, D], all contiguous
+ * and of one dtype. Products have float32 accuracy and the results one rounding; dk and
+ * dv are summed over the q heads of a KV head. Rows of no sequence, or past the first
+ * max_seq_len of theirs, get zeros. head_dim 1..128. Results do not depend on timing.
+ *   workspace: kvfp8_prefill_backward_workspace_bytes(...) bytes, 16-byte aligned, any
+ *   contents; `aligned`: q, k, v and grad_out are 16-byte aligned (fewer bytes then). dq, dk and dv are 16-byte aligned.
+ * Replaces the backward of reference src/torch_llm/kernals/flash_attention.py:213 onwards.
+ */
+int64_t kvfp8_prefill_backward_workspace_bytes(int dtype, int64_t total_tokens, int32_t num_q_heads,
+                                               int32_t num_kv_heads, int32_t head_dim, int32_t batch,
+                                               int32_t max_seq_len, int aligned);
+int kvfp8_prefill_attention_backward(const void* q_dev, const void* k_dev, const void* v_dev, const void* out_dev,
+                                     const float* lse_dev, const void* grad_out_dev, int dtype, int64_t total_tokens,
+                                     int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim,
+                                     const void* cu_seqlens_dev, int cu_dtype, int32_t batch, int32_t max_seq_len,
+                                     float scale, void* dq_dev, void* dk_dev, void* dv_dev,
+                                     void* workspace_dev, int64_t workspace_bytes, void* stream);
+
+/*
  * Fused append + decode: the quantize-and-scatter write of every sequence's new
  * token and the paged decode attention over the context that includes it, in the
  * decode kernel's launches (no separate append launch).

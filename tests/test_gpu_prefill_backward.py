@@ -1,0 +1,109 @@
+"""The HIP backward of the packed causal attention against float64 autograd, at the edges of
+its tiles (16 own rows, 32 streamed rows, 64 keys), its head-size and dtype variants, and
+its splits over q heads."""
+
+import math
+
+import pytest
+import torch as t
+
+from aiproj_amd.kernals import flash_attention as fa
+
+pytestmark = pytest.mark.gpu
+
+# The gradients are rounded once to their dtype (half an ulp: 2^-9 and 2^-12 relative, 2-norm
+# below that), and so are the saved output and lse they start from; float32 gradients carry
+# the forward's two-part 16-bit products (about 1e-5). Twice that.
+TOLERANCE = {t.bfloat16: 4e-3, t.float16: 5e-4, t.float32: 2e-5}
+
+
+def reference(q, k, v, bounds, longest, grad):
+    dq, dk, dv = (t.zeros(x.shape, dtype=t.float64, device=x.device) for x in (q, k, v))
+    groups = q.shape[1] // k.shape[1]
+    for s0, s1 in zip(bounds, bounds[1:]):
+        n = min(s1 - s0, longest)
+        rows = slice(s0, s0 + n)
+        if n == 0:
+            continue
+        ins = [x[rows].double().requires_grad_(True) for x in (q, k, v)]
+        qs, ks, vs = (x.transpose(0, 1) for x in ins)
+        ks, vs = ks.repeat_interleave(groups, 0), vs.repeat_interleave(groups, 0)
+        s = t.matmul(qs, ks.transpose(1, 2).contiguous()) / math.sqrt(q.shape[2])
+        s = s.masked_fill(t.ones(n, n, dtype=t.bool, device=q.device).triu(1), -math.inf)
+        out = t.matmul(t.softmax(s, -1), vs).transpose(0, 1)
+        for to, g in zip((dq, dk, dv), t.autograd.grad(out, ins, grad[rows].double())):
+            to[rows] = g
+    return dq, dk, dv
+
+
+def inputs(lengths, hq, hkv, d, dtype, seed=0, extra=0):
+    bounds = [0]
+    for n in lengths:
+        bounds.append(bounds[-1] + n)
+    gen = t.Generator(device="cuda").manual_seed(seed)
+    rows = [t.randn(bounds[-1] + extra, h, d, generator=gen, device="cuda").to(dtype) for h in (hq, hkv, hkv, hq)]
+    return bounds, rows
+
+
+def check(got, want, dtype):
+    for g, w in zip(got, want):
+        assert g.dtype == dtype
+        assert float((g.double() - w).norm()) <= TOLERANCE[dtype] * float(w.norm())
+
+
+@pytest.mark.parametrize("dtype", [t.bfloat16, t.float16, t.float32])
+@pytest.mark.parametrize("hq,hkv,d", [(4, 1, 128), (4, 2, 64), (3, 3, 96), (8, 2, 80), (2, 1, 17), (6, 2, 120)])
+def test_backward_matches_float64(dtype, hq, hkv, d):
+    lengths = [1, 15, 16, 17, 31, 32, 33, 0, 63, 64, 65, 127, 129, 200]
+    bounds, (q, k, v, grad) = inputs(lengths, hq, hkv, d, dtype, seed=d)
+    cu = t.tensor(bounds, dtype=t.int32, device="cuda")
+    scale = 1 / math.sqrt(d)
+    out, lse = fa.flash_attention_forward(q, k, v, cu, max(lengths), scale)
+    got = fa._native_backward(q, k, v, out, lse, cu, grad, max(lengths), scale)
+    assert got is not None
+    check(got, reference(q, k, v, bounds, max(lengths), grad), dtype)
+
+
+@pytest.mark.parametrize("count", [1, 8, 24])
+def test_backward_splits_over_q_heads(count):
+    """One long sequence to many: every number of workgroups per KV head, twice the same bits."""
+    lengths = [520] * count
+    bounds, (q, k, v, grad) = inputs(lengths, 8, 2, 64, t.bfloat16, seed=count)
+    cu = t.tensor(bounds, dtype=t.int64, device="cuda")
+    out, lse = fa.flash_attention_forward(q, k, v, cu, 520, 0.125)
+    got = fa._native_backward(q, k, v, out, lse, cu, grad, 520, 0.125)
+    check(got, reference(q, k, v, bounds, 520, grad), t.bfloat16)
+    again = fa._native_backward(q, k, v, out, lse, cu, grad, 520, 0.125)
+    assert all(t.equal(a, b) for a, b in zip(got, again))
+
+
+def test_rows_of_no_sequence_get_zeros():
+    """Rows past the last sequence, and rows past batch_max_seq_len of theirs."""
+    for hq in (2, 8):
+        bounds, (q, k, v, grad) = inputs([70, 40], hq, 2, 64, t.float16, extra=9)
+        cu = t.tensor(bounds, dtype=t.int32, device="cuda")
+        out, lse = fa.flash_attention_forward(q, k, v, cu, 50, 0.125)
+        got = fa._native_backward(q, k, v, out, lse, cu, grad, 50, 0.125)
+        check(got, reference(q, k, v, bounds, 50, grad), t.float16)
+        for g in got:
+            assert not g[50:70].any() and not g[110:].any()
+
+
+def test_unaligned_inputs_and_other_calls():
+    """Inputs off a 16-byte boundary are read through the planes; what the kernels do not take
+    keeps the PyTorch path."""
+    bounds, (q, k, v, grad) = inputs([33, 70], 4, 2, 64, t.bfloat16)
+    cu = t.tensor(bounds, dtype=t.int32, device="cuda")
+    out, lse = fa.flash_attention_forward(q, k, v, cu, 70, 0.125)
+    want = reference(q, k, v, bounds, 70, grad)
+
+    def shifted(x):
+        flat = t.empty(x.numel() + 1, dtype=x.dtype, device=x.device)
+        flat[1:] = x.flatten()
+        return flat[1:].view(x.shape)
+
+    got = fa._native_backward(shifted(q), shifted(k), shifted(v), shifted(out), lse, cu, shifted(grad), 70, 0.125)
+    check(got, want, t.bfloat16)
+    strided = grad.transpose(0, 1).contiguous().transpose(0, 1)
+    assert fa._native_backward(q, k, v, out, lse, cu, strided, 70, 0.125) is None
+    check(fa.flash_attention_backward(q, k, v, out, lse, cu, strided, 70, 0.125), want, t.bfloat16)
