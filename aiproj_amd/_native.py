@@ -53,6 +53,8 @@ SIGNATURES = {
     "kvfp8_rmsnorm_forward": (_INT, [_P, _INT, _I64, _I64, _I32, _P, _INT, ctypes.c_float, _P, _I64, _P, _P]),
     "kvfp8_add_rmsnorm_forward": (_INT, [_P, _P, _INT, _I64, _I64, _I64, _I32, _P, _INT, ctypes.c_float,
                                          _P, _I64, _P, _I64, _P, _P]),
+    "kvfp8_rmsnorm_backward_workspace_bytes": (_I64, [_I64, _I32]),
+    "kvfp8_rmsnorm_backward": (_INT, [_P, _P, _INT, _I64, _I64, _I64, _I32, _P, _INT, _P, _P, _I64, _P, _P, _I64, _P]),
     "kvfp8_rope_inplace": (_INT, [_P, _INT, _I64, _I32, _I32, _I64, _I64, _P, _INT, _P, _P, _INT, _I64, _P]),
     "kvfp8_silu_mul": (_INT, [_P, _INT, _I64, _I32, _I64, _P, _I64, _P]),
     "kvfp8_prefill_attention": (_INT, [_P, _P, _P, _INT, _I64, _I32, _I32, _I32, _P, _INT, _I32, _I32,

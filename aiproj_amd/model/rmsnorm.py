@@ -7,8 +7,9 @@ dtype, with `inv_rms = 1 / sqrt(mean(x^2) + eps)` per row.
 
 The forward runs the gfx950 HIP kernel `rmsnorm_kernel` through the C ABI
 `kvfp8_rmsnorm_forward`; `add_rmsnorm` is the residual add fused with the norm
-that follows it (`kvfp8_add_rmsnorm_forward`). The backward (training, outside
-this path) is written with PyTorch operations from the saved `inv_rms`.
+that follows it (`kvfp8_add_rmsnorm_forward`). The backward runs `rmsnorm_backward_kernel`
+(`kvfp8_rmsnorm_backward`) from the saved `inv_rms` for aligned rows of a multiple of 8 up
+to 4096 elements, and PyTorch float32 operations otherwise.
 """
 
 from __future__ import annotations
@@ -63,6 +64,30 @@ def add_rmsnorm(x: t.Tensor, update: t.Tensor, weight: t.Tensor, eps: float):
     return state, out
 
 
+def _native_backward(x, weight, inv_rms, grad_output):
+    """(dx, dw) from the HIP kernels, or None for what they do not take."""
+    if x.device.type != "cuda" or x.ndim != 2 or x.numel() == 0 or grad_output.dtype != x.dtype:
+        return None
+    d = x.shape[1]
+    weight = weight.contiguous()
+    grad_output = grad_output if grad_output.stride(1) == 1 else grad_output.contiguous()
+    size = 16 // x.element_size()
+    if (d % 8 or d > 4096 or x.stride(1) != 1 or x.stride(0) % size or grad_output.stride(0) % size
+            or any(y.data_ptr() % 16 for y in (x, weight, grad_output))):
+        return None
+    device = _native.require_gpu(x, weight, inv_rms, grad_output, what="rmsnorm")
+    nbytes = _native.lib().kvfp8_rmsnorm_backward_workspace_bytes(x.shape[0], d)
+    dx = t.empty_like(x, memory_format=t.contiguous_format)
+    dw = t.empty_like(weight)
+    workspace = t.empty(nbytes, dtype=t.uint8, device=x.device)
+    rc = _native.lib().kvfp8_rmsnorm_backward(
+        x.data_ptr(), grad_output.data_ptr(), _native.dtype_code(x.dtype), x.stride(0), grad_output.stride(0),
+        x.shape[0], d, weight.data_ptr(), _native.dtype_code(weight.dtype), inv_rms.data_ptr(),
+        dx.data_ptr(), dx.stride(0), dw.data_ptr(), workspace.data_ptr(), nbytes, _native.stream_handle(device))
+    _native.check(rc, "kvfp8_rmsnorm_backward")
+    return dx, dw
+
+
 class RMSNormFunction(t.autograd.Function):
     @staticmethod
     def forward(ctx, x, weight, eps):
@@ -74,6 +99,9 @@ class RMSNormFunction(t.autograd.Function):
     @t.autograd.function.once_differentiable
     def backward(ctx, grad_output):
         x, weight, inv_rms = ctx.saved_tensors
+        grads = _native_backward(x, weight, inv_rms, grad_output)
+        if grads is not None:
+            return *grads, None
         x32, g32, w32 = x.float(), grad_output.float(), weight.float()
         inv = inv_rms.unsqueeze(1)
         xhat = x32 * inv

@@ -217,6 +217,19 @@ int kvfp8_add_rmsnorm_forward(const void* x_dev, const void* update_dev, int dty
                               void* out_dev, int64_t out_stride, float* inv_rms_dev, void* stream);
 
 /*
+ * Backward of kvfp8_rmsnorm_forward in float32: dx (x's dtype) and dw (weight's dtype) from
+ * x, the forward's inv_rms and the gradient of its output (x's dtype). d_model: multiples of
+ * 8 up to 4096 (KVFP8_ELIMIT otherwise), rows 16-byte aligned. The workspace holds
+ * kvfp8_rmsnorm_backward_workspace_bytes(...) bytes, any contents. Sums are added in a fixed
+ * order. No reference counterpart on this path (training).
+ */
+int64_t kvfp8_rmsnorm_backward_workspace_bytes(int64_t rows, int32_t d_model);
+int kvfp8_rmsnorm_backward(const void* x_dev, const void* grad_dev, int dtype, int64_t x_stride, int64_t grad_stride,
+                           int64_t rows, int32_t d_model, const void* weight_dev, int w_dtype,
+                           const float* inv_rms_dev, void* dx_dev, int64_t dx_stride, void* dw_dev,
+                           void* workspace_dev, int64_t workspace_bytes, void* stream);
+
+/*
  * Varlen causal attention over packed prompts (prefill):
  *   q [T, Hq, D], k and v [T, Hkv, D] contiguous, one dtype (f32/f16/bf16);
  *   cu_seqlens [batch + 1] (int32/int64): sequence b is tokens
