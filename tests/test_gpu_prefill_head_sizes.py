@@ -1,0 +1,34 @@
+"""Head sizes 80, 96 and 112 on the eight-wave prompt-attention kernel, over its persistent
+workgroups, item edges and scales, against the oracle."""
+
+import math
+
+import numpy as np
+import pytest
+import torch as t
+
+import oracle
+from aiproj_amd.kernals.flash_attention import flash_attention_forward
+
+pytestmark = pytest.mark.gpu
+
+# One rounding of the output and of the probabilities to the type, as for head size 64.
+TOLERANCE = {t.float16: 2e-3, t.bfloat16: 1.6e-2}
+
+
+@t.inference_mode()
+@pytest.mark.parametrize("dtype", [t.float16, t.bfloat16])
+@pytest.mark.parametrize("head_dim", [80, 96, 112])
+@pytest.mark.parametrize("sign", [1, -1])
+def test_wide_kernel_head_sizes(dtype, head_dim, sign):
+    lengths = [1, 16, 31, 33, 63, 64, 65, 127, 129, 191, 257, 300] * 2
+    gen = t.Generator(device="cuda").manual_seed(head_dim)
+    q, k, v = (t.randn(sum(lengths), h, head_dim, device="cuda", generator=gen).to(dtype) for h in (8, 2, 2))
+    cu = t.tensor([0] + list(np.cumsum(lengths)), dtype=t.int32, device="cuda")
+    scale = sign / math.sqrt(head_dim)
+    out, lse = flash_attention_forward(q, k, v, cu, max(lengths), scale)
+    want, want_lse = oracle.causal_varlen_attention(*(x.double().cpu().numpy() for x in (q, k, v)), cu.cpu().numpy(),
+                                                    max(lengths), scale)
+    tol = TOLERANCE[dtype]
+    t.testing.assert_close(out.double().cpu(), t.from_numpy(want), rtol=tol, atol=tol)
+    t.testing.assert_close(lse.double().cpu(), t.from_numpy(want_lse), rtol=1e-3, atol=1e-3)
