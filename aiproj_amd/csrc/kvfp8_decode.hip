@@ -928,8 +928,9 @@ KernelTiming kvfp8::next_kernel_timing() {
 
 namespace {
 
-// Whether a call runs on the MFMA kernel: the plan allows it, the caches are
-// 16-byte aligned, an f16 cache comes with f16 q, and slot * 32 + count fits the
+// Whether a call runs on the MFMA kernel: the plan allows it (p.mfma, which paged_decode
+// clears for a narrow head size whose states do not fit the workspace at hand), the caches
+// are 16-byte aligned, an f16 cache comes with f16 q, and slot * 32 + count fits the
 // kernel's int32 per sequence.
 bool takes_mfma(const Plan& p, const void* k_cache, const void* v_cache, int64_t bt_rows, int q_dtype,
                 int kv_dtype) {
@@ -1037,7 +1038,7 @@ extern "C" int kvfp8_append_decode_supported(int32_t batch, int32_t num_q_heads,
         bt_width <= 0 || !pow2(block_size) || num_q_heads % num_kv_heads != 0)
         return 0;
     const Plan p = make_plan(batch, num_q_heads, num_kv_heads, head_dim, bt_width, block_size, kv_dtype);
-    return p.mfma && bt_rows < ((int64_t)1 << 26) ? 1 : 0;
+    return p.mfma && !narrow_head(head_dim) && bt_rows < ((int64_t)1 << 26) ? 1 : 0;
 }
 
 extern "C" int kvfp8_append_paged_decode(KVFP8_DECODE_PARAMS, const void* k_new, const void* v_new, int new_dtype,
@@ -1088,7 +1089,14 @@ int paged_decode(const void* q, int q_dtype, int64_t q_stride_b, int64_t q_strid
     if (!q || !k_cache || !v_cache || !block_table || !slots || !context_lengths || !out) return KVFP8_ENULL;
     if (kv_dtype == KVFP8_E4M3FN && (!k_scales || !v_scales)) return KVFP8_ENULL;
 
-    const Plan p = make_plan(batch, num_q_heads, num_kv_heads, head_dim, bt_width, block_size, kv_dtype);
+    Plan p = make_plan(batch, num_q_heads, num_kv_heads, head_dim, bt_width, block_size, kv_dtype);
+    if (p.mfma && narrow_head(head_dim)) {
+        // The vector-ALU kernels take these sizes too, with other states: a workspace (or the
+        // static scratch) that holds only theirs still serves the call. The fused append
+        // runs over whole rows only.
+        const int64_t have = use_scratch ? kScratchBytes : workspace_bytes;
+        if (fresh || workspace_taken(p, true, batch, num_q_heads, num_kv_heads, head_dim) > have) p.mfma = false;
+    }
     const bool mfma = takes_mfma(p, k_cache, v_cache, bt_rows, q_dtype, kv_dtype);
     const int64_t need = workspace_taken(p, mfma, batch, num_q_heads, num_kv_heads, head_dim);
     if (use_scratch) {

@@ -5,7 +5,11 @@
 
 namespace kvfp8 {
 
-// Shapes the MFMA kernel handles (e4m3fn, bf16 or f16 cache, D in {64, 128}, page
+// Head sizes that e4m3fn caches take in the layout of 128 (rows narrower than it): the
+// plain decode only.
+bool narrow_head(int32_t head_dim);
+
+// Shapes the MFMA kernel handles (e4m3fn, bf16 or f16 cache, D in {64, 128}, e4m3fn also narrow, page
 // size a multiple of 16, group size <= 16; an f16 cache also needs f16 q, which the
 // caller checks); everything else goes to the VALU kernels.
 bool mfma_decode_supported(int32_t batch, int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim,

@@ -2,7 +2,8 @@
 //
 // Replaces the Triton split and reduction kernels of reference
 // src/torch_llm/kernals/decode_attention.py:194-550 for e4m3fn and bf16 caches
-// (and f16 caches read with f16 q) with D in {64, 128} and pages of 16k tokens.
+// (and f16 caches read with f16 q) with D in {64, 128}, e4m3fn caches also with D in {80,
+// 96, 112}, and pages of 16k tokens.
 //
 // Work split. The attended tokens of the batch form one list of 16-token tiles
 // (sequence by sequence, tile prefix built in LDS from context_lengths, no host
@@ -137,9 +138,25 @@ __device__ __forceinline__ float row_ror8(float x) {
     return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x128, 0xF, 0xF, false));
 }
 
+// Narrow rows (kNarrow, C = 2): e4m3fn caches of head size 80, 96 or 112 in the layout of
+// 128. The head size is the caller's (d.head_dim, a multiple of 16); lanes whose dims lie
+// past it load the row's last ones again and their q operands are zero. These sizes keep the
+// precision of the vector-ALU kernels they would otherwise take: q and the probabilities
+// enter the products as bf16 parts that hold all of their bits, at most three. (bf16 and
+// f16 caches stay there: an infinite element would multiply parts that are zero.)
+// Measured, B 32, 512 to 4096 tokens, 32q/8kv heads, D 80, f16 q, append and decode: 66 us on
+// the vector ALU -> 41 us.
+//
 // The e4m3fn D = 128 kernel reads K in whole 128-byte rows (see load_step).
-template <int C, int ES>
-constexpr bool kWholeRowK = ES == 1 && C == 2;
+template <int C, int ES, bool kNarrow>
+constexpr bool kWholeRowK = ES == 1 && C == 2 && !kNarrow;
+
+// 16-bit parts of a q operand and of the probabilities: hi + lo for q that is not the operand
+// type, the probabilities with it. Narrow rows: as many as hold the float.
+template <int QT, bool kF16, bool kNarrow>
+constexpr int kQParts = QT == (kF16 ? KVFP8_F16 : KVFP8_BF16) ? 1 : (kNarrow && QT == KVFP8_F32 ? 3 : 2);
+template <int QT, bool kF16, bool kNarrow>
+constexpr int kPParts = kNarrow ? 3 : kQParts<QT, kF16, false>;
 
 // Token (within its 16-token tile, tile i / 4) of score i and V row i of lane group j.
 template <bool kWL>
@@ -226,10 +243,10 @@ struct StepData {
     float sc;                // e4m3fn: lane l holds the [k|v][tile A|B][token l % 16] scale
 };
 
-template <int C, int ES>
+template <int C, int ES, bool kNarrow>
 __device__ __forceinline__ void load_step(StepData<C, ES>& s, const MfmaArgs& a, int h, const TileRef& ta,
                                           const TileRef& tb, int lane) {
-    constexpr int D = 64 * C;
+    const int D = kNarrow ? a.d.head_dim : 64 * C;
     constexpr int NB = 4 * C;
     constexpr int KR = C * ES;
     constexpr int VW = C * ES;
@@ -240,8 +257,20 @@ __device__ __forceinline__ void load_step(StepData<C, ES>& s, const MfmaArgs& a,
     const int64_t eb = (tb.row0 * hkv + h) * D * ES;
     const uint8_t* kc = reinterpret_cast<const uint8_t*>(a.d.k_cache);
     const uint8_t* vc = reinterpret_cast<const uint8_t*>(a.d.v_cache);
-    constexpr bool kWL = kWholeRowK<C, ES>;
-    if constexpr (kWL) {
+    constexpr bool kWL = kWholeRowK<C, ES, kNarrow>;
+    if constexpr (kNarrow) {
+        // Token (l % 16), 16-byte runs at 64 r + 16 (l / 16), those past the row at its last
+        // run. Rows are no multiple of a cache line: normal loads, so that the line stays
+        // for the next head's wave. (A NaN code of the last run is in the score anyway.)
+        const uint32_t kbase = (uint32_t)(m16 * row_stride);
+#pragma unroll
+        for (int r = 0; r < KR; ++r) {
+            const int at = 64 * r + 16 * j;
+            const uint32_t koff = kbase + (uint32_t)min(at, D - 16);
+            s.ka[r] = *reinterpret_cast<const u32x4_t*>(kc + ea + koff);
+            s.kb[r] = *reinterpret_cast<const u32x4_t*>(kc + eb + koff);
+        }
+    } else if constexpr (kWL) {
         // Lane 2t + h + 16 j reads bytes 64 h + 16 j .. + 15 of token t (8 tokens
         // per instruction): every instruction reads eight whole 128-byte rows,
         // streamed with nontemporal loads.
@@ -267,11 +296,16 @@ __device__ __forceinline__ void load_step(StepData<C, ES>& s, const MfmaArgs& a,
             }
         }
     }
-    // Every V instruction reads whole rows (nontemporal).
+    // Every V instruction reads whole rows (nontemporal; narrow rows as K above).
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-        const uint8_t* p = vc + (i < 4 ? ea : eb) + (uint32_t)(step_token<kWL>(i, j) * row_stride + NB * ES * m16);
-        if constexpr (VW == 1) {
+        const int col = kNarrow ? min(NB * m16, D - NB) : NB * m16;
+        const uint8_t* p = vc + (i < 4 ? ea : eb) + (uint32_t)(step_token<kWL>(i, j) * row_stride + ES * col);
+        if constexpr (kNarrow) {
+            const u32x2_t y = *reinterpret_cast<const u32x2_t*>(p);
+            s.v[i][0] = y.x;
+            s.v[i][1] = y.y;
+        } else if constexpr (VW == 1) {
             s.v[i][0] = __builtin_nontemporal_load(reinterpret_cast<const uint32_t*>(p));
         } else if constexpr (VW == 2) {
             const u32x2_t x = __builtin_nontemporal_load(reinterpret_cast<const u32x2_t*>(p));
@@ -304,14 +338,14 @@ struct WaveState {
 // (c = l % 16, j = l / 16): the same permutation of the head dimension as the K
 // runs of load_step. Whole-row K: operand kb = 2 set + m holds column (g, h') =
 // c, head g = c % 8 + 8 set, dims of half h' = c / 8.
-template <int C, int ES>
+template <int C, int ES, bool kNarrow>
 __device__ __forceinline__ int qk_head(int kb, int c) {
-    if constexpr (kWholeRowK<C, ES>) return (c & 7) + 8 * (kb >> 1);
+    if constexpr (kWholeRowK<C, ES, kNarrow>) return (c & 7) + 8 * (kb >> 1);
     else return c;
 }
-template <int C, int ES>
+template <int C, int ES, bool kNarrow>
 __device__ __forceinline__ int qk_dim(int kb, int c, int j, int i) {
-    if constexpr (kWholeRowK<C, ES>) return 64 * (c >> 3) + 16 * j + 8 * (kb & 1) + i;
+    if constexpr (kWholeRowK<C, ES, kNarrow>) return 64 * (c >> 3) + 16 * j + 8 * (kb & 1) + i;
     else if constexpr (ES == 1) return 64 * (kb >> 1) + 16 * j + 8 * (kb & 1) + i;   // 16 codes per run, 2 MFMAs
     else return 32 * kb + 8 * j + i;                                                  // 8 values per run, 1 MFMA
 }
@@ -328,7 +362,7 @@ struct QRaw {
     uint32_t w[2 * C][kWords];
 };
 
-template <int C, int ES, int QT, int kOps>
+template <int C, int ES, int QT, int kOps, bool kNarrow>
 __device__ __forceinline__ void load_q_raw(const MfmaArgs& a, int b, int h, int G, int lane, QRaw<C, QT>& r) {
     using T = typename Elem<QT>::T;
     constexpr int kWords = QRaw<C, QT>::kWords;
@@ -337,8 +371,9 @@ __device__ __forceinline__ void load_q_raw(const MfmaArgs& a, int b, int h, int 
     const T* p[kOps];
 #pragma unroll
     for (int kb = 0; kb < kOps; ++kb) {
-        const int g = min(qk_head<C, ES>(kb, c), G - 1);
-        p[kb] = base + (int64_t)(h * G + g) * a.d.q_stride_h + qk_dim<C, ES>(kb, c, j, 0);
+        const int g = min(qk_head<C, ES, kNarrow>(kb, c), G - 1);
+        const int dim = qk_dim<C, ES, kNarrow>(kb, c, j, 0);
+        p[kb] = base + (int64_t)(h * G + g) * a.d.q_stride_h + (kNarrow ? min(dim, a.d.head_dim - 8) : dim);
     }
     if (a.q_vec) {
 #pragma unroll
@@ -366,16 +401,17 @@ __device__ __forceinline__ void load_q_raw(const MfmaArgs& a, int b, int h, int 
     }
 }
 
-// Q^T operands from the raw elements: bf16 (f32 and f16 q as hi + lo parts) or f16
-// (f16 q, exact), zero for heads g >= G and for operands not loaded.
-template <int C, int ES, int QT, int kOps, bool kHiLo, bool kF16>
-__device__ __forceinline__ void q_operands(const QRaw<C, QT>& r, int G, int lane, OpT<kF16>* qh, OpT<kF16>* ql) {
+// Q^T operands from the raw elements, in kParts parts (see kQParts): zero for heads g >= G,
+// for dims past the head size D and for operands not loaded.
+template <int C, int ES, int QT, int kOps, int kParts, bool kF16, bool kNarrow>
+__device__ __forceinline__ void q_operands(const QRaw<C, QT>& r, int G, int D, int lane, OpT<kF16> (*q)[2 * C]) {
     using E = OpE<kF16>;
     using T = typename Elem<QT>::T;
     const int c = lane & 15;
 #pragma unroll
     for (int kb = 0; kb < 2 * C; ++kb) {
-        const bool live = kb < kOps && qk_head<C, ES>(kb, c) < G;
+        const bool live = kb < kOps && qk_head<C, ES, kNarrow>(kb, c) < G &&
+                          (!kNarrow || qk_dim<C, ES, kNarrow>(kb, c, lane >> 4, 0) < D);
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
             float x = 0.0f;
@@ -384,17 +420,20 @@ __device__ __forceinline__ void q_operands(const QRaw<C, QT>& r, int G, int lane
                 else x = Elem<QT>::load((T)((r.w[kb][i >> 1] >> (16 * (i & 1))) & 0xFFFFu));
             }
             x = live ? x : 0.0f;
-            const E hi = (E)x;
-            qh[kb][i] = hi;
-            if constexpr (kHiLo) ql[kb][i] = (E)(x - (float)hi);
+#pragma unroll
+            for (int p = 0; p < kParts; ++p) {
+                const E hi = (E)x;
+                q[p][kb][i] = hi;
+                // (An infinite q is its first part alone.)
+                x = kNarrow && __builtin_isinf(x) ? 0.0f : x - (float)hi;
+            }
         }
     }
 }
 
-template <int C, int ES, bool kHiLo, int kSets, bool kF16>
-__device__ __forceinline__ void compute_step(WaveState<C>& st, const StepData<C, ES>& s, const OpT<kF16>* qh,
-                                             const OpT<kF16>* ql, float4* stage, int lane, int lim_a,
-                                             int lim_b, float score_scale) {
+template <int C, int ES, int kQP, int kPP, int kSets, bool kF16, bool kNarrow>
+__device__ __forceinline__ void compute_step(WaveState<C>& st, const StepData<C, ES>& s, const OpT<kF16> (*q)[2 * C],
+                                             float4* stage, int lane, int lim_a, int lim_b, float score_scale) {
     static_assert(!kF16 || ES == 2, "f16 operands come from an f16 cache");
     using Op = OpT<kF16>;
     using E = OpE<kF16>;
@@ -402,7 +441,7 @@ __device__ __forceinline__ void compute_step(WaveState<C>& st, const StepData<C,
     const int j = lane >> 4;
     const bool full = lim_a == 16 && lim_b == 16;   // wave-uniform
 
-    constexpr bool kWL = kWholeRowK<C, ES>;
+    constexpr bool kWL = kWholeRowK<C, ES, kNarrow>;
     // Per-token scales of score i (k, with sm_scale * log2(e)) and V row i (v).
     float ks[8], vs[8];
     if constexpr (ES == 1) {
@@ -460,20 +499,18 @@ __device__ __forceinline__ void compute_step(WaveState<C>& st, const StepData<C,
             const u32x4_t kr = x < 2 ? s.ka[x] : s.kb[x - 2];
             const bf16x8_t k0 = fp8x8(kr[0], kr[1]), k1 = fp8x8(kr[2], kr[3]);
             f32x4_t d0 = {0.0f, 0.0f, 0.0f, 0.0f};
-            d0 = mma(k0, qh[0], d0);
-            d0 = mma(k1, qh[1], d0);
-            if constexpr (kHiLo) {
-                d0 = mma(k0, ql[0], d0);
-                d0 = mma(k1, ql[1], d0);
+#pragma unroll
+            for (int p = 0; p < kQP; ++p) {
+                d0 = mma(k0, q[p][0], d0);
+                d0 = mma(k1, q[p][1], d0);
             }
             f32x4_t d1 = d0;
             if constexpr (kSets == 2) {
                 d1 = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-                d1 = mma(k0, qh[2], d1);
-                d1 = mma(k1, qh[3], d1);
-                if constexpr (kHiLo) {
-                    d1 = mma(k0, ql[2], d1);
-                    d1 = mma(k1, ql[3], d1);
+#pragma unroll
+                for (int p = 0; p < kQP; ++p) {
+                    d1 = mma(k0, q[p][2], d1);
+                    d1 = mma(k1, q[p][3], d1);
                 }
             }
 #pragma unroll
@@ -496,11 +533,10 @@ __device__ __forceinline__ void compute_step(WaveState<C>& st, const StepData<C,
                 ka = __builtin_bit_cast(Op, s.ka[kb]);
                 kbv = __builtin_bit_cast(Op, s.kb[kb]);
             }
-            sa = mma(ka, qh[kb], sa);
-            sb = mma(kbv, qh[kb], sb);
-            if constexpr (kHiLo) {
-                sa = mma(ka, ql[kb], sa);
-                sb = mma(kbv, ql[kb], sb);
+#pragma unroll
+            for (int p = 0; p < kQP; ++p) {
+                sa = mma(ka, q[p][kb], sa);
+                sb = mma(kbv, q[p][kb], sb);
             }
         }
 #pragma unroll
@@ -545,11 +581,16 @@ __device__ __forceinline__ void compute_step(WaveState<C>& st, const StepData<C,
         for (int i = 0; i < 8; ++i)
             if (!live[i]) pv[i] = 0.0f;
     }
-    Op ph, pl;
+    Op pp[kPP];
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-        ph[i] = (E)pv[i];
-        if constexpr (kHiLo) pl[i] = (E)(pv[i] - (float)ph[i]);
+        float x = pv[i];
+#pragma unroll
+        for (int p = 0; p < kPP; ++p) {
+            const E hi = (E)x;
+            pp[p][i] = hi;
+            x -= (float)hi;
+        }
     }
 
     // V rows: zero the rows of masked tokens (stale pages may hold NaN).
@@ -574,10 +615,10 @@ __device__ __forceinline__ void compute_step(WaveState<C>& st, const StepData<C,
                 e[3][p] = fp8x2_hi(y);
             }
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const bf16x8_t av = cat8(e[q][0], e[q][1], e[q][2], e[q][3]);
-                st.o[4 * c + q] = mma(av, ph, st.o[4 * c + q]);
-                if constexpr (kHiLo) st.o[4 * c + q] = mma(av, pl, st.o[4 * c + q]);
+            for (int x = 0; x < 4; ++x) {
+                const bf16x8_t av = cat8(e[x][0], e[x][1], e[x][2], e[x][3]);
+#pragma unroll
+                for (int p = 0; p < kPP; ++p) st.o[4 * c + x] = mma(av, pp[p], st.o[4 * c + x]);
             }
         }
     } else {
@@ -589,8 +630,8 @@ __device__ __forceinline__ void compute_step(WaveState<C>& st, const StepData<C,
 #pragma unroll
             for (int p = 0; p < 4; ++p) w[p] = __builtin_amdgcn_perm(vr[2 * p + 1][nb >> 1], vr[2 * p][nb >> 1], sel);
             const Op av = __builtin_bit_cast(Op, w);
-            st.o[nb] = mma(av, ph, st.o[nb]);
-            if constexpr (kHiLo) st.o[nb] = mma(av, pl, st.o[nb]);
+#pragma unroll
+            for (int p = 0; p < kPP; ++p) st.o[nb] = mma(av, pp[p], st.o[nb]);
         }
     }
 }
@@ -742,14 +783,13 @@ __device__ __forceinline__ void put_new_token(const MfmaArgs& a, const NewRow<C>
     }
 }
 
-template <int C, int QT, int ES, int kSets, bool kAppend, bool kF16, bool kRep>
+template <int C, int QT, int ES, int kSets, bool kAppend, bool kF16, bool kRep, bool kNarrow>
 __global__ void __launch_bounds__(kMaxThreads)
 decode_mfma_kernel(MfmaArgs a) {
-    constexpr int D = 64 * C;
+    static_assert(!kNarrow || (C == 2 && ES == 1 && !kAppend && kSets == 1), "narrow rows: the plain decode only");
+    const int D = kNarrow ? a.d.head_dim : 64 * C;
     constexpr int NB = 4 * C;
-    // q as bf16 hi + lo unless it is the operand type already (bf16 q on bf16
-    // operands, f16 q on f16 operands).
-    constexpr bool kHiLo = kF16 ? QT != KVFP8_F16 : QT != KVFP8_BF16;
+    constexpr int kQP = kQParts<QT, kF16, kNarrow>, kPP = kPParts<QT, kF16, kNarrow>;
     extern __shared__ int32_t prefix[];                // [batch + 1], then meta [batch]
     __shared__ int32_t wave_total[kMaxWaves];
     __shared__ float4 stage_all[kMaxWaves][16];
@@ -857,13 +897,16 @@ decode_mfma_kernel(MfmaArgs a) {
             // is computed, into the buffer step T - 2 used (three buffers), so step
             // T + 2 is in flight while T is computed and two steps while the wave
             // waits; bf16 steps are twice the bytes and keep one step in flight (two
-            // buffers).
+            // buffers), and so do narrow rows with f32 or f16 q (the parts of q
+            // take the registers: 70 and 13 spilled with three buffers; B 32 x 2000, 32q/8kv
+            // heads, D 80: 45 -> 30 us and 30 -> 29 us).
+            constexpr bool kThree = ES == 1 && !(kNarrow && QT != KVFP8_BF16);
             // Q^T operands of this head's G query heads: loads issued before the
             // first K/V loads, converted after them, so that the first step waits
             // for nothing else.
-            constexpr int kQOps = kWholeRowK<C, ES> ? 2 * kSets : 2 * C;
+            constexpr int kQOps = kWholeRowK<C, ES, kNarrow> ? 2 * kSets : 2 * C;
             QRaw<C, QT> qraw;
-            load_q_raw<C, ES, QT, kQOps>(a, b, h, G, lane, qraw);
+            load_q_raw<C, ES, QT, kQOps, kNarrow>(a, b, h, G, lane, qraw);
             const int hq = h * G + m16;     // output column of this lane
             const bool qlive = m16 < G;
 
@@ -872,27 +915,28 @@ decode_mfma_kernel(MfmaArgs a) {
             auto issue = [&](StepData<C, ES>& dst, int32_t tile0, TileRef& ra, TileRef& rb) {
                 ra = tile_ref(a, table_row, tile0);
                 rb = tile0 + 1 < t1 ? tile_ref(a, table_row, tile0 + 1) : TileRef{0, 0};
-                load_step<C, ES>(dst, a, h, ra, rb, lane);
+                load_step<C, ES, kNarrow>(dst, a, h, ra, rb, lane);
             };
             int32_t T = T0;
             if (!kRep || T < t1) issue(buf0, T, r0a, r0b);
-            if constexpr (ES == 1) {
+            if constexpr (kThree) {
                 if (T + dT < t1) issue(buf1, T + dT, r1a, r1b);
             }
             if constexpr (kAppend) {
                 if (append && !put_early) put_new_token<C>(a, fresh, lane);
             }
-            OpT<kF16> qh[2 * C], ql[2 * C];
-            q_operands<C, ES, QT, kQOps, kHiLo, kF16>(qraw, G, lane, qh, ql);
+            OpT<kF16> qp[kQP][2 * C];
+            q_operands<C, ES, QT, kQOps, kQP, kF16, kNarrow>(qraw, G, D, lane, qp);
 
 
             auto compute = [&](const StepData<C, ES>& cur, int32_t tile0, const TileRef& ra, const TileRef& rb) {
                 const int64_t pos = (int64_t)tile0 * 16;
                 const int lim_a = ra.valid ? (int)max((int64_t)0, min((int64_t)16, len - pos)) : 0;
                 const int lim_b = rb.valid ? (int)max((int64_t)0, min((int64_t)16, len - pos - 16)) : 0;
-                compute_step<C, ES, kHiLo, kSets, kF16>(st, cur, qh, ql, stage, lane, lim_a, lim_b, a.d.score_scale);
+                compute_step<C, ES, kQP, kPP, kSets, kF16, kNarrow>(st, cur, qp, stage, lane, lim_a, lim_b,
+                                                                    a.d.score_scale);
             };
-            if constexpr (ES == 1) {
+            if constexpr (kThree) {
                 while (!kRep || T < t1) {
                     compute(buf0, T, r0a, r0b);
                     if (T + 2 * dT < t1) issue(buf2, T + 2 * dT, r2a, r2b);
@@ -970,6 +1014,7 @@ decode_mfma_kernel(MfmaArgs a) {
                     const float inv = lt > 0.0f ? 1.0f / lt : 0.0f;
 #pragma unroll
                     for (int jj = 0; jj < 4; ++jj) {
+                        if (kNarrow && NB * (4 * j + jj) >= D) continue;
 #pragma unroll
                         for (int nb = 0; nb < NB; ++nb)
                             store_out<QT>(a.d, b, hq, NB * (4 * j + jj) + nb, lt > 0.0f ? st.o[nb][jj] * inv : 0.0f);
@@ -979,6 +1024,7 @@ decode_mfma_kernel(MfmaArgs a) {
                     float* acc = a.part_acc + pi * D;
 #pragma unroll
                     for (int jj = 0; jj < 4; ++jj) {
+                        if (kNarrow && NB * (4 * j + jj) >= D) continue;
 #pragma unroll
                         for (int nb = 0; nb < NB; ++nb) acc[NB * (4 * j + jj) + nb] = st.o[nb][jj];
                     }
@@ -1019,11 +1065,12 @@ __device__ __forceinline__ int32_t group_of(int64_t x, int64_t total, int64_t gr
 // One wave per (sequence, q head). Piece states are read lane-parallel (m and l
 // one piece per lane, acc as float4 runs with D/4 lanes per piece), so the merge
 // costs a couple of memory latencies whatever the number of pieces.
-template <int C, int QT>
+// Narrow rows take the lanes of 128 dims per piece; those past the row only follow.
+template <int C, int QT, bool kNarrow>
 __global__ void __launch_bounds__(256)
 combine_mfma_kernel(MfmaArgs a) {
-    constexpr int D = 64 * C;
-    constexpr int kLanesPerPiece = D / 4;
+    const int D = kNarrow ? a.d.head_dim : 64 * C;
+    constexpr int kLanesPerPiece = 16 * C;
     constexpr int kPiecesPerPass = 64 / kLanesPerPiece;
     // The wave index as a scalar, so that the per-sequence plan entries below are
     // scalar loads.
@@ -1035,7 +1082,7 @@ combine_mfma_kernel(MfmaArgs a) {
     const int32_t t0 = a.plan[b], t1 = a.plan[b + 1];
     const int d4 = lane % kLanesPerPiece, po = lane / kLanesPerPiece;
     if (t1 == t0) {
-        if (po == 0) store_out4<QT>(a.d, b, hq, 4 * d4, 0.0f, 0.0f, 0.0f, 0.0f);
+        if (po == 0 && (!kNarrow || 4 * d4 < D)) store_out4<QT>(a.d, b, hq, 4 * d4, 0.0f, 0.0f, 0.0f, 0.0f);
         return;
     }
     const int64_t total = a.plan[a.d.batch];
@@ -1063,7 +1110,7 @@ combine_mfma_kernel(MfmaArgs a) {
         const int64_t si = state_index(i);
         const float mi = a.part_m[si];
         const float li = a.part_l[si];
-        const float4 x = reinterpret_cast<const float4*>(a.part_acc + si * D)[d4];
+        const float4 x = reinterpret_cast<const float4*>(a.part_acc + si * D)[kNarrow ? min(d4, D / 4 - 1) : d4];
         const float mn = fmaxf(mr, mi);
         const float mu = mn == kNegInf ? 0.0f : mn;
         const float sa = fast_exp2(mr - mu), sb = fast_exp2(mi - mu);
@@ -1087,7 +1134,7 @@ combine_mfma_kernel(MfmaArgs a) {
         den = den * sa + __shfl_xor(den, off) * sb;
         mr = mn;
     }
-    if (po == 0) {
+    if (po == 0 && (!kNarrow || 4 * d4 < D)) {
         const bool ok = den > 0.0f;
         store_out4<QT>(a.d, b, hq, 4 * d4, ok ? num.x / den : 0.0f, ok ? num.y / den : 0.0f,
                        ok ? num.z / den : 0.0f, ok ? num.w / den : 0.0f);
@@ -1142,7 +1189,7 @@ int64_t max_groups(int32_t num_kv_heads) {
     return (int64_t)device_cus() * (per_cu > 0 ? per_cu : 1);
 }
 
-template <int C, int QT, int ES, int kSets, bool kAppend, bool kF16, bool kRep>
+template <int C, int QT, int ES, int kSets, bool kAppend, bool kF16, bool kRep, bool kNarrow>
 hipError_t launch_w(const MfmaArgs& a, int64_t cap, hipStream_t s, int phases) {
     const int threads = 64 * (kRep ? kMaxWaves : waves_for(a.d.num_kv_heads));
     const size_t lds = (size_t)(2 * a.d.batch + 1) * sizeof(int32_t) + (kRep ? replica_merge_bytes<C>() : 0);
@@ -1156,7 +1203,7 @@ hipError_t launch_w(const MfmaArgs& a, int64_t cap, hipStream_t s, int phases) {
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 0;
     int& per_cu = resident[dev][threads / 64];
     if (per_cu == 0) {
-        const void* fn = reinterpret_cast<const void*>(&decode_mfma_kernel<C, QT, ES, kSets, kAppend, kF16, kRep>);
+        const void* fn = reinterpret_cast<const void*>(&decode_mfma_kernel<C, QT, ES, kSets, kAppend, kF16, kRep, kNarrow>);
         int n = 0;
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, fn, threads, 0) != hipSuccess || n <= 0) n = 1;
         per_cu = n;
@@ -1173,31 +1220,33 @@ hipError_t launch_w(const MfmaArgs& a, int64_t cap, hipStream_t s, int phases) {
     groups = groups < cap ? groups : cap;
     if (phases & kPhaseSplit) {
         const hipError_t err =
-            launch_timed(decode_mfma_kernel<C, QT, ES, kSets, kAppend, kF16, kRep>, dim3((unsigned)groups),
+            launch_timed(decode_mfma_kernel<C, QT, ES, kSets, kAppend, kF16, kRep, kNarrow>, dim3((unsigned)groups),
                          dim3(threads), lds, s, next_kernel_timing(), a);
         if (err != hipSuccess) return err;
     }
     if (!(phases & kPhaseReduce)) return hipSuccess;
     const int64_t pairs = (int64_t)a.d.batch * a.d.num_q_heads;
-    hipLaunchKernelGGL((combine_mfma_kernel<C, QT>), dim3((unsigned)((pairs + 3) / 4)), dim3(256), 0, s, a);
+    hipLaunchKernelGGL((combine_mfma_kernel<C, QT, kNarrow>), dim3((unsigned)((pairs + 3) / 4)), dim3(256), 0, s, a);
     return hipGetLastError();
 }
 
-template <int C, int QT, int ES, int kSets, bool kAppend = false, bool kF16 = false>
+template <int C, int QT, int ES, int kSets, bool kAppend = false, bool kF16 = false, bool kNarrow = false>
 hipError_t launch_c(const MfmaArgs& a, int64_t cap, hipStream_t s, int phases) {
     if constexpr (!kAppend) {
         if (replicated<C>(a.d, (size_t)(2 * a.d.batch + 1) * sizeof(int32_t)))
-            return launch_w<C, QT, ES, kSets, kAppend, kF16, true>(a, cap, s, phases);
+            return launch_w<C, QT, ES, kSets, kAppend, kF16, true, kNarrow>(a, cap, s, phases);
     }
-    return launch_w<C, QT, ES, kSets, kAppend, kF16, false>(a, cap, s, phases);
+    return launch_w<C, QT, ES, kSets, kAppend, kF16, false, kNarrow>(a, cap, s, phases);
 }
 
 }  // namespace
 
+bool narrow_head(int32_t head_dim) { return head_dim == 80 || head_dim == 96 || head_dim == 112; }
+
 bool mfma_decode_supported(int32_t batch, int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim,
                            int64_t bt_width, int32_t block_size, int kv_dtype) {
     if (kv_dtype != KVFP8_E4M3FN && kv_dtype != KVFP8_BF16 && kv_dtype != KVFP8_F16) return false;
-    if (head_dim != 64 && head_dim != 128) return false;
+    if (head_dim != 64 && head_dim != 128 && !(narrow_head(head_dim) && kv_dtype == KVFP8_E4M3FN)) return false;
     if (block_size < 16 || block_size % 16 != 0) return false;
     if (num_q_heads % num_kv_heads != 0 || num_q_heads / num_kv_heads > 16) return false;
     if (num_kv_heads > kMaxWaves && num_kv_heads % kMaxWaves != 0) return false;
@@ -1243,6 +1292,7 @@ hipError_t launch_mfma_decode(const DecodeArgs& d, int kv_dtype, void* workspace
     const int64_t qsize = QT == KVFP8_F32 ? 4 : 2;
     a.q_vec = ((uintptr_t)d.q % 16 == 0 && (d.q_stride_b * qsize) % 16 == 0 && (d.q_stride_h * qsize) % 16 == 0) ? 1 : 0;
     const int64_t cap = max_groups(d.num_kv_heads);
+    if (narrow_head(d.head_dim)) return launch_c<2, QT, 1, 1, false, false, true>(a, cap, stream, phases);
     if (kv_dtype == KVFP8_BF16)
         return d.head_dim == 64 ? launch_c<1, QT, 2, 1>(a, cap, stream, phases)
                                 : launch_c<2, QT, 2, 1>(a, cap, stream, phases);

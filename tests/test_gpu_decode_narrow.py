@@ -1,0 +1,121 @@
+"""Decode at head sizes 80, 96 and 112 on the MFMA kernel (the layout of 128 with narrow
+rows), against float64 attention over the stored cache, and its fallback when a workspace
+holds only the vector-ALU kernels' states."""
+
+import math
+
+import pytest
+import torch as t
+
+from aiproj_amd import _native
+from aiproj_amd.inference.paged_kv_cache import PagedKVCache
+from aiproj_amd.kernals.decode_attention import PagedKVRead, decode_attention_wrapper, prepare_decode
+
+pytestmark = pytest.mark.gpu
+
+
+def batch(lengths, hq, hkv, d, cache_dtype, q_dtype, seed=0, page=16, poison=True):
+    gen = t.Generator(device="cuda").manual_seed(seed + d)
+    need = [-(-n // page) for n in lengths]
+    order = t.randperm(sum(need) + 2, generator=t.Generator().manual_seed(seed)).tolist()
+    table = t.full((len(lengths), max(need) + 1), -1, dtype=t.int32)
+    at = 0
+    for b, n in enumerate(need):
+        table[b, :n] = t.tensor(order[at:at + n], dtype=t.int32)
+        at += n
+    cache = PagedKVCache(sum(need) + 2, page, hkv, d, "cuda", cache_dtype)
+    # Unwritten slots hold NaN: nothing of them may reach an output.
+    for x in (cache.k, cache.v):
+        if cache.quantized:
+            x.view(t.uint8).fill_(0x7F)
+        else:
+            x.fill_(math.nan)
+    if cache.quantized:
+        cache.k_scales.fill_(math.nan)
+        cache.v_scales.fill_(math.nan)
+    pos = t.cat([t.arange(n) for n in lengths])
+    row = t.repeat_interleave(t.arange(len(lengths)), t.tensor(lengths))
+    blocks = table[row, pos // page].long().cuda()
+    offsets = (pos % page).cuda()
+    k, v = (t.randn(len(pos), hkv, d, generator=gen, device="cuda") for _ in range(2))
+    cache.append_kv(blocks, offsets, k, v)
+    q = t.randn(len(lengths), hq, d, generator=gen, device="cuda").to(q_dtype)
+    kv = PagedKVRead(cache.k, cache.v, cache.k_scales, cache.v_scales, table.cuda(),
+                     t.arange(len(lengths), device="cuda"), t.tensor(lengths, dtype=t.int32, device="cuda"), page)
+
+    def stored(x, scales):
+        rows = x[blocks, offsets].double()
+        return rows if scales is None else rows * scales[blocks, offsets].double().unsqueeze(-1)
+
+    return q, kv, stored(cache.k, cache.k_scales), stored(cache.v, cache.v_scales)
+
+
+def reference(q, k, v, lengths):
+    out, at, groups = t.zeros(q.shape, dtype=t.float64, device="cuda"), 0, q.shape[1] // k.shape[1]
+    for b, n in enumerate(lengths):
+        ks, vs = (x[at:at + n].transpose(0, 1).contiguous() for x in (k, v))
+        at += n
+        if n:
+            s = t.matmul(q[b].double().view(-1, groups, q.shape[2]), ks.transpose(1, 2).contiguous())
+            out[b] = t.matmul(t.softmax(s / math.sqrt(q.shape[2]), -1), vs).view(q.shape[1:])
+    return out
+
+
+# The output's rounding (half an ulp, 2-norm below 0.6 of it) over float32 arithmetic.
+TOLERANCE = {t.bfloat16: 2.5e-3, t.float16: 3.2e-4, t.float32: 2e-6}
+
+
+@pytest.mark.parametrize("q_dtype,cache_dtype", [
+    (t.bfloat16, t.float8_e4m3fn), (t.float16, t.float8_e4m3fn), (t.float32, t.float8_e4m3fn),
+    (t.float16, t.bfloat16)])
+@pytest.mark.parametrize("hq,hkv,d", [(32, 8, 80), (4, 2, 96), (16, 1, 112), (3, 3, 80)])
+def test_narrow_heads_match_float64(q_dtype, cache_dtype, hq, hkv, d):
+    lengths = [1, 15, 16, 17, 31, 32, 33, 0, 64, 65, 100, 257, 700, 1500]
+    q, kv, k, v = batch(lengths, hq, hkv, d, cache_dtype, q_dtype)
+    out = decode_attention_wrapper(q, kv)
+    want = reference(q, k, v, lengths)
+    assert not out[7].any()
+    assert float((out.double() - want).norm()) <= TOLERANCE[q_dtype] * float(want.norm())
+
+
+def test_narrow_heads_split_over_the_grid():
+    """Enough tokens for every workgroup (and replicas at two KV heads), pages of 32."""
+    for hq, hkv in ((32, 8), (8, 2)):
+        lengths = [9000, 4097, 1, 8191] + [700] * 20
+        q, kv, k, v = batch(lengths, hq, hkv, 80, t.float8_e4m3fn, t.bfloat16, page=32)
+        out = decode_attention_wrapper(q, kv)
+        want = reference(q, k, v, lengths)
+        assert float((out.double() - want).norm()) <= TOLERANCE[t.bfloat16] * float(want.norm())
+        assert t.equal(out, decode_attention_wrapper(q, kv))
+
+
+def test_infinite_values_stay_in_their_row():
+    """An infinite q element gives infinite scores, not NaN from its zero parts."""
+    lengths = [40, 40]
+    q, kv, k, v = batch(lengths, 4, 2, 80, t.float8_e4m3fn, t.float32)
+    # All of head 0's products with this q element are negative: no token is attended less
+    # than -inf, so only an exact split gives -inf (zero weights) and no NaN there.
+    q[0, 0, 79] = math.inf
+    k_neg = -(kv.k[:, :, 0, 79].float().abs())
+    kv.k[:, :, 0, 79] = t.where(k_neg == 0, -0.5, k_neg).to(t.float8_e4m3fn)
+    out = decode_attention_wrapper(q, kv)
+    want = reference(q, k, v, lengths)
+    assert not bool(t.isnan(out[0, 0]).any())          # no attended token: zeros, as before
+    rest = t.ones(4, dtype=t.bool, device="cuda")
+    rest[:2] = False                                    # heads 0 and 1 read the changed K
+    assert float((out[:, rest].double() - want[:, rest]).norm()) <= 2e-6 * float(want[:, rest].norm())
+
+
+def test_workspace_of_the_other_kernels_still_serves():
+    lengths = [20, 33]
+    q, kv, k, v = batch(lengths, 8, 2, 80, t.float8_e4m3fn, t.float32)
+    call = prepare_decode(q, kv)
+    chunks = -(-kv.block_table.shape[1] * 16 // 256)
+    states = len(lengths) * chunks * 8
+    small = 2 * (-(-states * 4 // 256) * 256) + (-(-states * 80 * 4 // 256) * 256)
+    assert small < call.workspace.numel()
+    args = list(call.args)
+    args[-2] = small
+    assert _native.lib().kvfp8_paged_decode(*args) == 0
+    want = reference(q, k, v, lengths)
+    assert float((call.output.double() - want).norm()) <= 2e-6 * float(want.norm())
