@@ -1,0 +1,250 @@
+// y = x W^T for the few rows of a decode step: x [M, K] with M <= 64, W [N, K] row-major (a
+// Linear layer's weight), bf16 or f16, float32 sums, one rounding.
+//
+// Bound: HBM, the weight read once (a decode step's weights exceed the last-level cache).
+//
+// Work split. A workgroup's eight waves divide K: wave w owns STEPS steps of 32 and the
+// workgroup walks over tiles of 16 weight rows. Everything a wave reads is a stream of
+// blocks of 16 rows of its K slice: first x (16 MT rows, kept in registers as MFMA operands:
+// 32 MT VGPRs at 8 steps), then its slice of tile after tile. Blocks go straight from global
+// memory into the wave's own two LDS slots, whole 512-byte row pieces per instruction (an
+// operand-shaped load of 64 bytes from each of 16 rows moved 25 bytes/ns per CU, from L2 as
+// from HBM: 64 rows through a 3072 x 2048 weight 12.4 us), one block in flight while the
+// other is used, with no barrier. The eight partial tiles meet in LDS and are added in
+// wave order. K beyond 2048 goes in groups, x read again. With fewer tiles than CUs the rows
+// of x are divided over workgroups instead (their second read of a tile hits L2).
+//
+// Measured (us, bf16, weights from HBM; 64 rows, then 1 row; in brackets torch's GEMM):
+//   3072 x 2048    8.0 [11.9]   5.4 [11.3]      2048 x 5632   12.0 [18.7]    9.2 [11.7]
+//   2048 x 2048    6.0 [11.6]   4.9 [11.0]     32000 x 2048   34.2 [36.0]   27.4 [34.9]
+//  11264 x 2048   16.5 [18.1]  12.2 [16.4]      8192 x 4096   26.7 [20.2]   16.0 [17.1]
+// The last one reads x twice per tile and has more tiles than workgroups: callers leave
+// such shapes (K above 2048 and more than 256 tiles) to the GEMM.
+#include "mfma_tiles.h"
+
+namespace kvfp8 {
+
+namespace {
+
+constexpr int kLinWaves = 8;
+constexpr int kLinSteps = 8;                 // K steps of 32 per wave and group
+constexpr int kLinRows = 16;                 // weight rows per tile
+
+struct LinArgs {
+    const uint8_t* x;
+    const uint8_t* w;
+    uint8_t* y;
+    int64_t x_row, y_row, w_row;             // bytes between rows
+    int32_t rows, tiles, steps;              // rows of x, tiles of N, K / 32
+    int32_t groups;                          // ceil(steps / (8 waves x steps per wave))
+    int32_t walkers;                         // workgroups that walk the tiles side by side
+};
+
+// Barrier over LDS accesses only: __syncthreads would also wait for the block in flight.
+__device__ __forceinline__ void lds_barrier() {
+    __asm__ volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    __asm__ volatile("" ::: "memory");
+}
+
+template <int MT, int STEPS, bool kF16>
+__global__ void __launch_bounds__(64 * kLinWaves, 2)
+skinny_linear_kernel(LinArgs a) {
+    constexpr int ROW = STEPS * 64;                  // bytes of a row's slice
+    constexpr int CPR = ROW / 16;                    // 16-byte chunks of it
+    constexpr int MASK = CPR < 16 ? CPR - 1 : 15;    // chunk c of row r sits in slot c ^ (r & MASK)
+    constexpr int BLOCK = 16 * ROW;
+    constexpr int LOADS = BLOCK / 1024;              // instructions per block
+    __shared__ __attribute__((aligned(16))) uint8_t ring[kLinWaves][2][BLOCK];
+    __shared__ __attribute__((aligned(16))) float sums[kLinWaves][MT * 16 * kLinRows];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int m16 = lane & 15, j = lane >> 4;
+    const int part = blockIdx.x / a.walkers, first = blockIdx.x % a.walkers;
+    const int m0 = part * 16 * MT;                   // this workgroup's rows of x
+    if (first >= a.tiles) return;
+
+    typedef __attribute__((address_space(3))) void* lds_ptr;
+    typedef __attribute__((address_space(3))) const uint8_t lds_u8;
+    typedef __attribute__((address_space(3))) const u32x4_t lds_u32x4;
+    const uint32_t ring0 = (uint32_t)(uintptr_t)(lds_ptr)&ring[wave][0][0];
+
+    // One block: rows row0 .. row0 + 15 (at most last_row) of a matrix, this wave's slice of
+    // group `group`; chunks past K repeat its last one (and are not multiplied).
+    // Instruction i fills 1 KB: slot lane of it is row (64 i + lane) / CPR. Inline assembly,
+    // waited for by hand, as in the prompt-attention kernel.
+    auto load = [&](const uint8_t* base, int64_t stride, int row0, int last_row, int group, int slot)
+        __attribute__((always_inline)) {
+        const int chunk0 = (group * kLinWaves + wave) * CPR;
+#pragma unroll
+        for (int i = 0; i < LOADS; ++i) {
+            const int r = (64 * i + lane) / CPR, c = (lane % CPR) ^ (r & MASK);
+            const uint8_t* p = base + min(row0 + r, last_row) * stride + 16 * (int64_t)min(chunk0 + c, 4 * a.steps - 1);
+            __asm__ volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off"
+                             :: "s"(__builtin_amdgcn_readfirstlane(ring0 + slot * BLOCK + 1024 * i)), "v"(p) : "memory");
+        }
+    };
+    // Operand of step s from a slot: row m16, chunk 4 s + j.
+    auto operand = [&](int slot, int s) __attribute__((always_inline)) -> u32x4_t {
+        return *(lds_u32x4*)(lds_u8*)(uintptr_t)(ring0 + slot * BLOCK + m16 * ROW + 16 * ((4 * s + j) ^ (m16 & MASK)));
+    };
+
+    // The stream: for each tile and group, the MT blocks of x (once when there is one
+    // group), then the tile's. The load cursor runs one block ahead.
+    int l_tile = first, l_group = 0, l_block = 0, l_slot = 0;
+    bool l_more = true;
+    auto load_next = [&]() __attribute__((always_inline)) -> bool {
+        if (!l_more) return false;
+        if (l_block < MT) load(a.x, a.x_row, m0 + 16 * l_block, a.rows - 1, l_group, l_slot);
+        else load(a.w, a.w_row, kLinRows * l_tile, kLinRows * a.tiles - 1, l_group, l_slot);
+        l_slot ^= 1;
+        if (++l_block <= MT) return true;
+        l_block = a.groups > 1 ? 0 : MT;
+        if (++l_group == a.groups) {
+            l_group = 0;
+            l_tile += a.walkers;
+            l_more = l_tile < a.tiles;
+        }
+        return true;
+    };
+    // The oldest block has arrived (`younger`: one more was issued after it); its slot may be
+    // filled again once its reads are done.
+    auto arrived = [&](bool younger) __attribute__((always_inline)) {
+        if (younger) __builtin_amdgcn_s_waitcnt((LOADS & 15) | (7 << 4) | (15 << 8));
+        else __builtin_amdgcn_s_waitcnt((7 << 4) | (15 << 8));
+        __asm__ volatile("" ::: "memory");
+    };
+    auto reads_done = [&]() __attribute__((always_inline)) {
+        __asm__ volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    };
+
+    u32x4_t x[MT][STEPS];
+    f32x4_t acc[MT];
+    int slot = 0;
+    load_next();
+    for (int tile = first; tile < a.tiles; tile += a.walkers) {
+        for (int group = 0; group < a.groups; ++group) {
+            if (a.groups > 1 || tile == first) {
+#pragma unroll
+                for (int t = 0; t < MT; ++t) {
+                    arrived(load_next());
+#pragma unroll
+                    for (int s = 0; s < STEPS; ++s) x[t][s] = operand(slot, s);
+                    reads_done();
+                    slot ^= 1;
+                }
+            }
+            arrived(load_next());
+            if (group == 0) {
+#pragma unroll
+                for (int t = 0; t < MT; ++t) acc[t] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+            }
+            const int valid = a.steps - (group * kLinWaves + wave) * STEPS;
+#pragma unroll
+            for (int s = 0; s < STEPS; ++s) {
+                if (s >= valid) break;       // wave-uniform
+                const u32x4_t w = operand(slot, s);
+#pragma unroll
+                for (int t = 0; t < MT; ++t) acc[t] = mma16<kF16>(w, x[t][s], acc[t]);
+            }
+            reads_done();
+            slot ^= 1;
+        }
+        // acc[t]: lane holds weight rows 4 j .. + 3 of x row 16 t + m16.
+#pragma unroll
+        for (int t = 0; t < MT; ++t)
+            *reinterpret_cast<f32x4_t*>(&sums[wave][(16 * t + m16) * kLinRows + 4 * j]) = acc[t];
+        lds_barrier();
+        // Thread: two neighbouring outputs of one row of x.
+        constexpr int kPairs = MT * 16 * kLinRows / 2;
+        if ((int)threadIdx.x < kPairs) {
+            const int at = 2 * threadIdx.x, row = m0 + at / kLinRows;
+            float2 sum = *reinterpret_cast<const float2*>(&sums[0][at]);
+#pragma unroll
+            for (int v = 1; v < kLinWaves; ++v) {
+                const float2 y = *reinterpret_cast<const float2*>(&sums[v][at]);
+                sum.x += y.x;
+                sum.y += y.y;
+            }
+            if (row < a.rows)
+                *reinterpret_cast<uint32_t*>(a.y + row * a.y_row + (int64_t)(tile * kLinRows + at % kLinRows) * 2) =
+                    pack2<kF16>(sum.x, sum.y);
+        }
+        lds_barrier();
+    }
+}
+
+int linear_cus() {
+    static int cus[64] = {};
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 0;
+    if (cus[dev] == 0) {
+        int n = 0;
+        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
+        cus[dev] = n;
+    }
+    return cus[dev];
+}
+
+template <int MT, int STEPS>
+hipError_t launch_linear(const LinArgs& a, bool f16, int grid, hipStream_t s) {
+    if (f16) hipLaunchKernelGGL((skinny_linear_kernel<MT, STEPS, true>), dim3(grid), dim3(64 * kLinWaves), 0, s, a);
+    else hipLaunchKernelGGL((skinny_linear_kernel<MT, STEPS, false>), dim3(grid), dim3(64 * kLinWaves), 0, s, a);
+    return hipGetLastError();
+}
+
+template <int MT>
+hipError_t launch_linear_steps(const LinArgs& a, int per_wave, bool f16, int grid, hipStream_t s) {
+    switch (per_wave) {
+        case 2: return launch_linear<MT, 2>(a, f16, grid, s);
+        case 4: return launch_linear<MT, 4>(a, f16, grid, s);
+        default: return launch_linear<MT, 8>(a, f16, grid, s);
+    }
+}
+
+}  // namespace
+
+}  // namespace kvfp8
+
+using namespace kvfp8;
+
+extern "C" int kvfp8_skinny_linear(const void* x, int dtype, int64_t x_stride, int32_t rows, int32_t k,
+                                   const void* weight, int64_t w_stride, int32_t n, void* out, int64_t out_stride,
+                                   void* stream) {
+    if (dtype != KVFP8_BF16 && dtype != KVFP8_F16) return KVFP8_EDTYPE;
+    if (rows < 0 || rows > 64 || k <= 0 || k % 32 != 0 || n <= 0 || n % kLinRows != 0) return KVFP8_ESHAPE;
+    if (rows == 0) return KVFP8_OK;
+    if (!x || !weight || !out) return KVFP8_ENULL;
+    if ((((uintptr_t)x | (uintptr_t)weight) & 15) != 0 || ((uintptr_t)out & 3) != 0 || x_stride % 8 != 0 ||
+        w_stride % 8 != 0 || out_stride % 2 != 0 || w_stride < k)
+        return KVFP8_ESTRIDE;
+    LinArgs a;
+    a.x = reinterpret_cast<const uint8_t*>(x);
+    a.w = reinterpret_cast<const uint8_t*>(weight);
+    a.y = reinterpret_cast<uint8_t*>(out);
+    a.x_row = x_stride * 2;
+    a.w_row = w_stride * 2;
+    a.y_row = out_stride * 2;
+    a.rows = rows;
+    a.tiles = n / kLinRows;
+    a.steps = k / 32;
+    int per_wave = 2;
+    while (per_wave < kLinSteps && kLinWaves * per_wave < a.steps) per_wave *= 2;
+    a.groups = (a.steps + kLinWaves * per_wave - 1) / (kLinWaves * per_wave);
+    const int cus = linear_cus();
+    // Row tiles per workgroup: all of them, or fewer while that puts idle CUs to work.
+    int mt = (rows + 15) / 16;
+    const int row_tiles = mt;
+    while (mt > 1 && (int64_t)a.tiles * ((row_tiles + mt / 2 - 1) / (mt / 2)) <= cus) mt /= 2;
+    const int parts = (row_tiles + mt - 1) / mt;
+    a.walkers = cus / parts < 1 ? 1 : cus / parts;
+    if (a.walkers > a.tiles) a.walkers = a.tiles;
+    hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+    const bool f16 = dtype == KVFP8_F16;
+    const int grid = a.walkers * parts;
+    switch (mt) {
+        case 1: return (int)launch_linear_steps<1>(a, per_wave, f16, grid, s);
+        case 2: return (int)launch_linear_steps<2>(a, per_wave, f16, grid, s);
+        case 3: return (int)launch_linear_steps<3>(a, per_wave, f16, grid, s);
+        default: return (int)launch_linear_steps<4>(a, per_wave, f16, grid, s);
+    }
+}

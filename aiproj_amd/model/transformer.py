@@ -22,7 +22,8 @@ What runs where: the norms (`rmsnorm_kernel`, residual add fused into the next
 norm), RoPE, the SwiGLU activation, the cache write and the decode attention are this
 library's HIP kernels (in decode, the new token's quantized write is done by the decode
 kernel itself);
-the projections and the FFN are plain GEMMs (hipBLASLt through torch); prompt
+the projections and the FFN are `RowLinear`: the HIP kernel `skinny_linear_kernel` for the
+few rows of a decode step, plain GEMMs (hipBLASLt through torch) otherwise; prompt
 (prefill) attention is the varlen causal HIP kernel behind `flash_attention_forward`,
 as the reference calls its FlashAttentionFunction there (`attention.py:103-110`).
 """
@@ -104,6 +105,51 @@ class RoPE(nn.Module):
         return x
 
 
+_SKINNY_ROWS = 64
+_SKINNY_TILES = 256       # weight tiles of 16 rows
+
+
+def _plain(x: t.Tensor) -> bool:
+    """A tensor whose address is its data: no transform, mode or trace looks at the operation."""
+    return (type(x) in (t.Tensor, nn.Parameter) and not t._C._functorch.is_functorch_wrapped_tensor(x)
+            and not t.compiler.is_compiling() and not t.jit.is_tracing() and t._C._len_torch_dispatch_stack() == 0
+            and t._C._len_torch_function_stack() == 0 and t.autograd.forward_ad._current_level < 0
+            and not t.is_autocast_enabled())
+
+
+def row_linear(x: t.Tensor, weight: t.Tensor) -> t.Tensor:
+    """x weight^T. Up to 64 rows of a 16-bit type without gradients run on the HIP kernel
+    `skinny_linear_kernel` (C ABI `kvfp8_skinny_linear`), everything else on torch's GEMM.
+    The kernel reads x again for each group of 2048 of K, so longer rows are left to the GEMM
+    unless a workgroup has one weight tile only."""
+    n, k = weight.shape
+    if (x.ndim != 2 or not 0 < x.shape[0] <= _SKINNY_ROWS or x.device.type != "cuda" or x.device != weight.device
+            or x.dtype not in (t.bfloat16, t.float16) or weight.dtype != x.dtype or x.shape[1] != k
+            or k % 32 or n % 16 or (k > 2048 and n // 16 > _SKINNY_TILES)
+            or (t.is_grad_enabled() and (x.requires_grad or weight.requires_grad))
+            or x.stride(1) != 1 or weight.stride(1) != 1 or x.stride(0) % 8 or weight.stride(0) % 8
+            or not _plain(x) or not _plain(weight) or x.data_ptr() % 16 or weight.data_ptr() % 16):
+        return F.linear(x, weight)
+    from aiproj_amd import _native
+
+    out = t.empty((x.shape[0], n), dtype=x.dtype, device=x.device)
+    rc = _native.lib().kvfp8_skinny_linear(x.data_ptr(), _native.dtype_code(x.dtype), x.stride(0), x.shape[0], k,
+                                           weight.data_ptr(), weight.stride(0), n, out.data_ptr(), n,
+                                           _native.stream_handle(x.device))
+    _native.check(rc, "kvfp8_skinny_linear")
+    return out
+
+
+class RowLinear(nn.Linear):
+    """nn.Linear without bias whose forward is `row_linear`."""
+
+    def __init__(self, in_features: int, out_features: int):
+        super().__init__(in_features, out_features, bias=False)
+
+    def forward(self, x: t.Tensor) -> t.Tensor:
+        return row_linear(x, self.weight)
+
+
 class Attention(nn.Module):
     def __init__(self, cfg: ModelConfig):
         super().__init__()
@@ -111,8 +157,8 @@ class Attention(nn.Module):
         self.q_dim = cfg.num_q_heads * cfg.head_dim
         self.kv_dim = cfg.num_kv_heads * cfg.head_dim
         # q, k and v projections as one GEMM (the reference's three Linear layers, concatenated).
-        self.qkv_proj = nn.Linear(cfg.d_model, self.q_dim + 2 * self.kv_dim, bias=False)
-        self.o_proj = nn.Linear(self.q_dim, cfg.d_model, bias=False)
+        self.qkv_proj = RowLinear(cfg.d_model, self.q_dim + 2 * self.kv_dim)
+        self.o_proj = RowLinear(self.q_dim, cfg.d_model)
         self.rope = RoPE(cfg.head_dim, cfg.max_seq_len, cfg.rope_theta)
 
     def forward(self, h: t.Tensor, meta: StepMeta, cache) -> t.Tensor:
@@ -157,8 +203,8 @@ class SwiGLU(nn.Module):
     def __init__(self, cfg: ModelConfig):
         super().__init__()
         self.d_ff = cfg.d_ff
-        self.gate_up = nn.Linear(cfg.d_model, 2 * cfg.d_ff, bias=False)
-        self.down = nn.Linear(cfg.d_ff, cfg.d_model, bias=False)
+        self.gate_up = RowLinear(cfg.d_model, 2 * cfg.d_ff)
+        self.down = RowLinear(cfg.d_ff, cfg.d_model)
 
     def forward(self, h: t.Tensor) -> t.Tensor:
         return self.down(silu_mul(self.gate_up(h), self.d_ff))
@@ -208,4 +254,4 @@ class TransformerLM(nn.Module):
             # Only the last prompt token of each sequence is sampled from.
             last = meta.cu_seqlens[1:].long() - 1
             h = h[last]
-        return F.linear(h, self.embed.weight)
+        return row_linear(h, self.embed.weight)

@@ -357,6 +357,16 @@ int kvfp8_silu_mul(const void* x_dev, int dtype, int64_t rows, int32_t n, int64_
 int kvfp8_timing_enable(int32_t max_launches);
 int kvfp8_timing_read(double* total_ms, int64_t* launches);
 
+/*
+ * out [rows, n] = x [rows, k] weight^T for the few rows of a decode step: weight [n, k]
+ * row-major, everything one dtype (f16/bf16), float32 sums, one rounding. rows 0..64, k a
+ * multiple of 32, n of 16; x and weight rows 16-byte aligned. Strides in elements. The
+ * projections of reference src/torch_llm/model/attention.py:57-122 and its FFN at M <= 64.
+ */
+int kvfp8_skinny_linear(const void* x_dev, int dtype, int64_t x_stride, int32_t rows, int32_t k,
+                        const void* weight_dev, int64_t w_stride, int32_t n, void* out_dev, int64_t out_stride,
+                        void* stream);
+
 /* Human-readable name of a return code (negative KVFP8_E* or positive hipError_t). */
 const char* kvfp8_strerror(int code);
 

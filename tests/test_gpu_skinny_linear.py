@@ -1,0 +1,56 @@
+"""The decode-step GEMM (few rows) against float64, at the edges of its tiles, K slices, K
+groups and row splits, and the calls that stay on torch's GEMM."""
+
+import pytest
+import torch as t
+
+from aiproj_amd.model import transformer
+from aiproj_amd.model.transformer import RowLinear, row_linear
+
+pytestmark = pytest.mark.gpu
+
+
+# Weight tiles: one, one short of a round of 256 workgroups, several rounds. K: one step,
+# slices of 2, 4 and 8 steps that end inside, at and past a wave's, groups of 2048.
+@t.no_grad()
+@pytest.mark.parametrize("dtype", [t.bfloat16, t.float16])
+@pytest.mark.parametrize("rows", [1, 15, 16, 17, 33, 48, 64])
+@pytest.mark.parametrize("n,k", [(16, 32), (48, 96), (4080, 256), (2048, 544), (4112, 1024), (272, 2016), (9008, 2048),
+                                 (2048, 5632), (512, 2080), (4096, 4128)])
+def test_matches_float64(dtype, rows, n, k, monkeypatch):
+    gen = t.Generator(device="cuda").manual_seed(rows * n + k)
+    x = t.randn(rows, k + 8, generator=gen, device="cuda").to(dtype)[:, :k]     # rows with a stride
+    w = (t.randn(n, k, generator=gen, device="cuda") / k ** 0.5).to(dtype)
+    want = x.double() @ w.double().T
+    monkeypatch.setattr(transformer.F, "linear", None)                          # the kernel, nothing else
+    out = row_linear(x, w)
+    assert out.dtype == dtype and out.shape == (rows, n)
+    # One rounding of the output over exact products and float32 sums: half an ulp, which is
+    # at most 2^-8 of a bf16 value (8-bit significand) and 2^-11 of an f16 one; the sums' own
+    # error (about 1e-6 of the terms) shows where they cancel.
+    half_ulp = 2.0 ** -8 if dtype == t.bfloat16 else 2.0 ** -11
+    t.testing.assert_close(out.double(), want, rtol=half_ulp, atol=1e-5)
+    assert t.equal(out, row_linear(x, w))
+    # A row's result does not depend on the rows beside it.
+    assert t.equal(out[rows // 2], row_linear(x[rows // 2:rows // 2 + 1], w)[0])
+
+
+def test_other_calls_stay_on_torch(monkeypatch):
+    calls = []
+    linear = transformer.F.linear
+    monkeypatch.setattr(transformer.F, "linear", lambda x, w: calls.append(1) or linear(x, w))
+    layer = RowLinear(64, 32).to("cuda", t.bfloat16)
+    x = t.randn(4, 64, device="cuda", dtype=t.bfloat16)
+    layer(x).sum().backward()                                  # gradients
+    assert len(calls) == 1 and layer.weight.grad is not None
+    with t.no_grad():
+        layer(x)
+        assert len(calls) == 1                                 # the kernel
+        layer(x.expand(2, 4, 64))
+        layer(x[:0])
+        layer(t.randn(65, 64, device="cuda", dtype=t.bfloat16))
+        layer.float()(x.float())
+        row_linear(x, t.randn(24, 64, device="cuda", dtype=t.bfloat16))
+        assert len(calls) == 6
+        t.func.vmap(lambda a: row_linear(a, t.ones(32, 64, device="cuda", dtype=t.bfloat16)))(x[None])
+        assert len(calls) == 7
