@@ -20,6 +20,7 @@ LIBRARY_PATH = Path(__file__).resolve().parent / "libkvfp8.so"
 
 # enum kvfp8_dtype in include/kvfp8.h
 F32, F16, BF16, E4M3FN, I32, I64 = 0, 1, 2, 3, 4, 5
+ESTRIDE = -3       # KVFP8_ESTRIDE: an unsupported stride or alignment
 ELIMIT = -6        # KVFP8_ELIMIT: a size beyond what the kernels support
 
 TORCH_TO_CODE = {
@@ -56,6 +57,7 @@ SIGNATURES = {
     "kvfp8_rmsnorm_backward_workspace_bytes": (_I64, [_I64, _I32]),
     "kvfp8_rmsnorm_backward": (_INT, [_P, _P, _INT, _I64, _I64, _I64, _I32, _P, _INT, _P, _P, _I64, _P, _P, _I64, _P]),
     "kvfp8_rope_inplace": (_INT, [_P, _INT, _I64, _I32, _I32, _I64, _I64, _P, _INT, _P, _P, _INT, _I64, _P]),
+    "kvfp8_rope_split": (_INT, [_P, _INT, _I64, _I32, _I32, _I32, _I64, _P, _INT, _P, _P, _INT, _I64, _P, _P, _P, _P]),
     "kvfp8_skinny_linear": (_INT, [_P, _INT, _I64, _I32, _I32, _P, _I64, _I32, _P, _I64, _P]),
     "kvfp8_silu_mul": (_INT, [_P, _INT, _I64, _I32, _I64, _P, _I64, _P]),
     "kvfp8_prefill_attention": (_INT, [_P, _P, _P, _INT, _I64, _I32, _I32, _I32, _P, _INT, _I32, _I32,

@@ -104,6 +104,26 @@ class RoPE(nn.Module):
         _native.check(rc, "kvfp8_rope_inplace")
         return x
 
+    def split(self, qkv: t.Tensor, positions: t.Tensor, num_q_heads: int, num_kv_heads: int):
+        """Packed q and k (rotated) and v of fused projection rows [q heads | k heads | v heads],
+        one launch of `rope_vec_kernel`; None for rows it does not take."""
+        from aiproj_amd import _native
+
+        device = _native.require_gpu(qkv, positions, what="rope")
+        if qkv.stride(-1) != 1 or not self.cos_table.is_contiguous():
+            raise ValueError("rope: rows need unit element stride")
+        q, k, v = (t.empty((qkv.shape[0], heads, self.head_dim), dtype=qkv.dtype, device=qkv.device)
+                   for heads in (num_q_heads, num_kv_heads, num_kv_heads))
+        rc = _native.lib().kvfp8_rope_split(
+            qkv.data_ptr(), _native.dtype_code(qkv.dtype), qkv.shape[0], num_q_heads, num_kv_heads, self.head_dim,
+            qkv.stride(0), positions.data_ptr(), _native.dtype_code(positions.dtype), self.cos_table.data_ptr(),
+            self.sin_table.data_ptr(), _native.dtype_code(self.cos_table.dtype), self.cos_table.shape[0],
+            q.data_ptr(), k.data_ptr(), v.data_ptr(), _native.stream_handle(device))
+        if rc == _native.ESTRIDE:
+            return None
+        _native.check(rc, "kvfp8_rope_split")
+        return q, k, v
+
 
 _SKINNY_ROWS = 64
 _SKINNY_TILES = 256       # weight tiles of 16 rows
@@ -164,12 +184,20 @@ class Attention(nn.Module):
     def forward(self, h: t.Tensor, meta: StepMeta, cache) -> t.Tensor:
         cfg = self.cfg
         qkv = self.qkv_proj(h)
+        ctx = meta.cache_context
+        if meta.mode == "prefill":
+            # Prompt attention takes packed q, k and v: rotated and split in one pass.
+            split = self.rope.split(qkv, meta.token_positions, cfg.num_q_heads, cfg.num_kv_heads)
+            if split is not None:
+                q, k, v = split
+                out, _ = flash_attention_forward(q, k, v, meta.cu_seqlens, meta.max_seqlen, 1.0 / math.sqrt(cfg.head_dim))
+                cache.append_kv(ctx.physical_blocks, ctx.block_offsets, k, v)
+                return self.o_proj(out.reshape(-1, self.q_dim))
         # q and k heads are the first Hq + Hkv heads of every row: one in-place rotation.
         self.rope.apply_(qkv, meta.token_positions, cfg.num_q_heads + cfg.num_kv_heads)
         q = qkv[:, :self.q_dim].view(-1, cfg.num_q_heads, cfg.head_dim)
         k = qkv[:, self.q_dim:self.q_dim + self.kv_dim].view(-1, cfg.num_kv_heads, cfg.head_dim)
         v = qkv[:, self.q_dim + self.kv_dim:].view(-1, cfg.num_kv_heads, cfg.head_dim)
-        ctx = meta.cache_context
         if meta.mode == "prefill":
             # The varlen causal HIP kernel (reference FlashAttentionFunction, `attention.py:103-110`).
             # q, k and v are views into the fused projection; the kernel takes packed rows.

@@ -337,6 +337,17 @@ int kvfp8_rope_inplace(void* x_dev, int dtype, int64_t rows, int32_t heads, int3
                        int64_t table_rows, void* stream);
 
 /*
+ * kvfp8_rope_inplace's rotation of the fused projection rows [q heads | k heads | v heads]
+ * (head_dim elements each), written to packed q [rows, num_q_heads, head_dim], k and v
+ * [rows, num_kv_heads, head_dim]; v is copied. head_dim a multiple of 8, rows, tables and
+ * outputs aligned for 16-byte accesses (KVFP8_ESTRIDE otherwise).
+ */
+int kvfp8_rope_split(const void* x_dev, int dtype, int64_t rows, int32_t num_q_heads, int32_t num_kv_heads,
+                     int32_t head_dim, int64_t row_stride, const void* positions_dev, int pos_dtype,
+                     const void* cos_table_dev, const void* sin_table_dev, int table_dtype, int64_t table_rows,
+                     void* q_out_dev, void* k_out_dev, void* v_out_dev, void* stream);
+
+/*
  * SwiGLU activation: out[r, j] = silu(g) * u with g = x[r, j], u = x[r, n + j] and
  * silu(g) = g * (1 / (1 + exp(-g))), in float32 with one rounding to the dtype
  * (f32/f16/bf16). x rows hold gate then up (row stride >= 2 n elements); out rows
