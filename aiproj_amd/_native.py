@@ -173,6 +173,17 @@ def stream_handle(device: torch.device) -> int:
     return torch.cuda.current_stream(device).cuda_stream
 
 
+def is_plain(*tensors: torch.Tensor) -> bool:
+    """Tensors whose addresses are their data: no vmap or other transform, mode or trace looks
+    at the operation, which a kernel called with addresses would hide from it."""
+    if (torch.compiler.is_compiling() or torch.jit.is_tracing() or torch._C._len_torch_dispatch_stack()
+            or torch._C._len_torch_function_stack() or torch.autograd.forward_ad._current_level >= 0):
+        return False
+    wrapped = torch._C._functorch.is_functorch_wrapped_tensor
+    return all(type(x) in (torch.Tensor, torch.nn.Parameter) and torch._C._has_storage(x) and not wrapped(x)
+               for x in tensors)
+
+
 def require_gpu(*tensors, what: str) -> torch.device:
     """All tensors on one GPU device; the FP8 path has no CPU implementation. The common
     case compares device indices (get_device: -1 on the CPU) without building device

@@ -69,6 +69,8 @@ _MAX_BACKWARD_HEAD = 128
 def _native_backward(q, k, v, output, lse, cum_seq, grad_output, batch_max_seq_len, scale):
     """dq, dk, dv from the HIP kernels, or None for what they do not take."""
     rows = (q, k, v, output, grad_output)
+    if not _native.is_plain(*rows, lse, cum_seq):
+        return None
     if (q.device.type != "cuda" or q.dtype not in _DTYPES or q.ndim != 3 or q.shape[2] > _MAX_BACKWARD_HEAD
             or q.numel() == 0 or lse.dtype != t.float32 or cum_seq.dtype not in (t.int32, t.int64) or cum_seq.ndim != 1
             or cum_seq.shape[0] < 2 or not 0 < int(batch_max_seq_len) < 2 ** 31):

@@ -66,7 +66,8 @@ def add_rmsnorm(x: t.Tensor, update: t.Tensor, weight: t.Tensor, eps: float):
 
 def _native_backward(x, weight, inv_rms, grad_output):
     """(dx, dw) from the HIP kernels, or None for what they do not take."""
-    if x.device.type != "cuda" or x.ndim != 2 or x.numel() == 0 or grad_output.dtype != x.dtype:
+    if (x.device.type != "cuda" or x.ndim != 2 or x.numel() == 0 or grad_output.dtype != x.dtype
+            or not _native.is_plain(x, weight, inv_rms, grad_output)):
         return None
     d = x.shape[1]
     weight = weight.contiguous()

@@ -129,29 +129,22 @@ _SKINNY_ROWS = 64
 _SKINNY_TILES = 256       # weight tiles of 16 rows
 
 
-def _plain(x: t.Tensor) -> bool:
-    """A tensor whose address is its data: no transform, mode or trace looks at the operation."""
-    return (type(x) in (t.Tensor, nn.Parameter) and not t._C._functorch.is_functorch_wrapped_tensor(x)
-            and not t.compiler.is_compiling() and not t.jit.is_tracing() and t._C._len_torch_dispatch_stack() == 0
-            and t._C._len_torch_function_stack() == 0 and t.autograd.forward_ad._current_level < 0
-            and not t.is_autocast_enabled())
-
-
 def row_linear(x: t.Tensor, weight: t.Tensor) -> t.Tensor:
     """x weight^T. Up to 64 rows of a 16-bit type without gradients run on the HIP kernel
     `skinny_linear_kernel` (C ABI `kvfp8_skinny_linear`), everything else on torch's GEMM.
     The kernel reads x again for each group of 2048 of K, so longer rows are left to the GEMM
     unless a workgroup has one weight tile only."""
+    from aiproj_amd import _native
+
     n, k = weight.shape
     if (x.ndim != 2 or not 0 < x.shape[0] <= _SKINNY_ROWS or x.device.type != "cuda" or x.device != weight.device
             or x.dtype not in (t.bfloat16, t.float16) or weight.dtype != x.dtype or x.shape[1] != k
-            or k % 32 or n % 16 or (k > 2048 and n // 16 > _SKINNY_TILES)
+            or not n or not k or k % 32 or n % 16 or (k > 2048 and n // 16 > _SKINNY_TILES)
             or (t.is_grad_enabled() and (x.requires_grad or weight.requires_grad))
             or x.stride(1) != 1 or weight.stride(1) != 1 or x.stride(0) % 8 or weight.stride(0) % 8
-            or not _plain(x) or not _plain(weight) or x.data_ptr() % 16 or weight.data_ptr() % 16):
+            or weight.stride(0) < k or t.is_autocast_enabled()
+            or not _native.is_plain(x, weight) or x.data_ptr() % 16 or weight.data_ptr() % 16):
         return F.linear(x, weight)
-    from aiproj_amd import _native
-
     out = t.empty((x.shape[0], n), dtype=x.dtype, device=x.device)
     rc = _native.lib().kvfp8_skinny_linear(x.data_ptr(), _native.dtype_code(x.dtype), x.stride(0), x.shape[0], k,
                                            weight.data_ptr(), weight.stride(0), n, out.data_ptr(), n,

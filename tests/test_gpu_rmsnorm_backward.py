@@ -34,3 +34,18 @@ def test_native_backward_leaves_other_rows_to_pytorch():
     assert rmsnorm_module._native_backward(x, w, t.ones(6, device="cuda"), x) is None       # not a multiple of 8
     x = t.randn(6, 65, device="cuda")[:, 1:]
     assert rmsnorm_module._native_backward(x, w.new_ones(64), t.ones(6, device="cuda"), x) is None   # unaligned rows
+
+
+def test_batched_gradients_take_pytorch():
+    """vmap over the backward (is_grads_batched) sees PyTorch operations, equal to one backward per gradient."""
+    gen = t.Generator(device="cuda").manual_seed(3)
+    x, w = t.randn(5, 64, generator=gen, device="cuda"), t.randn(64, generator=gen, device="cuda")
+    grads = t.randn(3, 5, 64, generator=gen, device="cuda")
+    x.requires_grad_(True)
+    w.requires_grad_(True)
+    out = rmsnorm_module.RMSNormFunction.apply(x, w, 1e-5)
+    got = t.autograd.grad(out, (x, w), grads, retain_graph=True, is_grads_batched=True)
+    for i in range(3):
+        # float32 sums of 64 terms and fewer in two orders.
+        for a, b in zip(got, t.autograd.grad(out, (x, w), grads[i], retain_graph=True)):
+            assert float((a[i] - b).norm()) <= 1e-5 * float(b.norm())
