@@ -173,4 +173,10 @@ struct RowDivider {
     KVFP8_HD float divide(float x) const { return fast ? corrected(x) : x / scale; }
 };
 
+// silu(gate) * up.
+__device__ __forceinline__ float swiglu(float g, float u) {
+    const float s = 1.0f / (1.0f + expf(-g));
+    return (g * s) * u;
+}
+
 }  // namespace kvfp8

@@ -14,11 +14,6 @@ namespace kvfp8 {
 
 constexpr int kSwigluThreads = 256;
 
-__device__ __forceinline__ float swiglu(float g, float u) {
-    const float s = 1.0f / (1.0f + expf(-g));
-    return (g * s) * u;
-}
-
 template <int DT, bool VEC>
 __global__ void __launch_bounds__(kSwigluThreads)
 silu_mul_kernel(const void* x, int64_t rows, int32_t n, int64_t x_stride, void* out, int64_t out_stride) {

@@ -129,28 +129,38 @@ _SKINNY_ROWS = 64
 _SKINNY_TILES = 256       # weight tiles of 16 rows
 
 
-def row_linear(x: t.Tensor, weight: t.Tensor) -> t.Tensor:
-    """x weight^T. Up to 64 rows of a 16-bit type without gradients run on the HIP kernel
-    `skinny_linear_kernel` (C ABI `kvfp8_skinny_linear`), everything else on torch's GEMM.
-    The kernel reads x again for each group of 2048 of K, so longer rows are left to the GEMM
-    unless a workgroup has one weight tile only."""
+def _takes_skinny(x: t.Tensor, weight: t.Tensor) -> bool:
+    """Up to 64 rows of a 16-bit type without gradients. The kernel reads x again for each group
+    of 2048 of K, so longer rows are left to the GEMM unless a workgroup has one weight tile only."""
     from aiproj_amd import _native
 
     n, k = weight.shape
-    if (x.ndim != 2 or not 0 < x.shape[0] <= _SKINNY_ROWS or x.device.type != "cuda" or x.device != weight.device
-            or x.dtype not in (t.bfloat16, t.float16) or weight.dtype != x.dtype or x.shape[1] != k
-            or not n or not k or k % 32 or n % 16 or (k > 2048 and n // 16 > _SKINNY_TILES)
-            or (t.is_grad_enabled() and (x.requires_grad or weight.requires_grad))
-            or x.stride(1) != 1 or weight.stride(1) != 1 or x.stride(0) % 8 or weight.stride(0) % 8
-            or weight.stride(0) < k or t.is_autocast_enabled()
-            or not _native.is_plain(x, weight) or x.data_ptr() % 16 or weight.data_ptr() % 16):
-        return F.linear(x, weight)
-    out = t.empty((x.shape[0], n), dtype=x.dtype, device=x.device)
-    rc = _native.lib().kvfp8_skinny_linear(x.data_ptr(), _native.dtype_code(x.dtype), x.stride(0), x.shape[0], k,
-                                           weight.data_ptr(), weight.stride(0), n, out.data_ptr(), n,
-                                           _native.stream_handle(x.device))
-    _native.check(rc, "kvfp8_skinny_linear")
+    return not (x.ndim != 2 or not 0 < x.shape[0] <= _SKINNY_ROWS or x.device.type != "cuda" or x.device != weight.device
+                or x.dtype not in (t.bfloat16, t.float16) or weight.dtype != x.dtype or x.shape[1] != k
+                or not n or not k or k % 32 or n % 16 or (k > 2048 and n // 16 > _SKINNY_TILES)
+                or (t.is_grad_enabled() and (x.requires_grad or weight.requires_grad))
+                or x.stride(1) != 1 or weight.stride(1) != 1 or x.stride(0) % 8 or weight.stride(0) % 8
+                or weight.stride(0) < k or t.is_autocast_enabled()
+                or not _native.is_plain(x, weight) or x.data_ptr() % 16 or weight.data_ptr() % 16)
+
+
+def _skinny(entry: str, x: t.Tensor, weight: t.Tensor, columns: int) -> t.Tensor:
+    from aiproj_amd import _native
+
+    out = t.empty((x.shape[0], columns), dtype=x.dtype, device=x.device)
+    rc = getattr(_native.lib(), entry)(x.data_ptr(), _native.dtype_code(x.dtype), x.stride(0), x.shape[0], x.shape[1],
+                                       weight.data_ptr(), weight.stride(0), columns, out.data_ptr(), columns,
+                                       _native.stream_handle(x.device))
+    _native.check(rc, entry)
     return out
+
+
+def row_linear(x: t.Tensor, weight: t.Tensor) -> t.Tensor:
+    """x weight^T: the HIP kernel `skinny_linear_kernel` (C ABI `kvfp8_skinny_linear`) for what
+    `_takes_skinny` names, torch's GEMM otherwise."""
+    if not _takes_skinny(x, weight):
+        return F.linear(x, weight)
+    return _skinny("kvfp8_skinny_linear", x, weight, weight.shape[0])
 
 
 class RowLinear(nn.Linear):
@@ -161,6 +171,12 @@ class RowLinear(nn.Linear):
 
     def forward(self, x: t.Tensor) -> t.Tensor:
         return row_linear(x, self.weight)
+
+    def unobserved(self) -> bool:
+        """Whether calling the layer does nothing but its own forward: no hook sees its output."""
+        hooks = nn.modules.module
+        return not (type(self) is not RowLinear or "forward" in self.__dict__ or self._forward_hooks
+                    or self._forward_pre_hooks or hooks._global_forward_hooks or hooks._global_forward_pre_hooks)
 
 
 class Attention(nn.Module):
@@ -228,7 +244,12 @@ class SwiGLU(nn.Module):
         self.down = RowLinear(cfg.d_ff, cfg.d_model)
 
     def forward(self, h: t.Tensor) -> t.Tensor:
-        return self.down(silu_mul(self.gate_up(h), self.d_ff))
+        up = self.gate_up
+        # A decode step's activation is done by the projection's kernel (`kvfp8_skinny_linear_swiglu`).
+        if (isinstance(up, RowLinear) and up.unobserved() and up.weight.shape[0] == 2 * self.d_ff
+                and _takes_skinny(h, up.weight)):
+            return self.down(_skinny("kvfp8_skinny_linear_swiglu", h, up.weight, self.d_ff))
+        return self.down(silu_mul(up(h), self.d_ff))
 
 
 class DecoderLayer(nn.Module):

@@ -378,6 +378,15 @@ int kvfp8_skinny_linear(const void* x_dev, int dtype, int64_t x_stride, int32_t 
                         const void* weight_dev, int64_t w_stride, int32_t n, void* out_dev, int64_t out_stride,
                         void* stream);
 
+/*
+ * out [rows, n] = silu(x G^T) * (x U^T) with weight [2 n, k] the rows of G then those of U:
+ * kvfp8_skinny_linear followed by kvfp8_silu_mul, bit for bit, in one launch. n a multiple of
+ * 8, the rest as kvfp8_skinny_linear.
+ */
+int kvfp8_skinny_linear_swiglu(const void* x_dev, int dtype, int64_t x_stride, int32_t rows, int32_t k,
+                               const void* weight_dev, int64_t w_stride, int32_t n, void* out_dev,
+                               int64_t out_stride, void* stream);
+
 /* Human-readable name of a return code (negative KVFP8_E* or positive hipError_t). */
 const char* kvfp8_strerror(int code);
 

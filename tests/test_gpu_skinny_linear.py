@@ -5,7 +5,7 @@ import pytest
 import torch as t
 
 from aiproj_amd.model import transformer
-from aiproj_amd.model.transformer import RowLinear, row_linear
+from aiproj_amd.model.transformer import ModelConfig, RowLinear, SwiGLU, row_linear, silu_mul
 
 pytestmark = pytest.mark.gpu
 
@@ -54,3 +54,24 @@ def test_other_calls_stay_on_torch(monkeypatch):
         assert len(calls) == 6
         t.func.vmap(lambda a: row_linear(a, t.ones(32, 64, device="cuda", dtype=t.bfloat16)))(x[None])
         assert len(calls) == 7
+
+
+# One tile, a tile more than a round of 256 workgroups, rows divided over workgroups, K groups.
+@t.no_grad()
+@pytest.mark.parametrize("dtype", [t.bfloat16, t.float16])
+@pytest.mark.parametrize("rows", [1, 17, 33, 64])
+@pytest.mark.parametrize("d_ff,k", [(8, 32), (2056, 96), (520, 1024), (5632, 2048), (1024, 2080)])
+def test_gated_projection_equals_the_two_launches(dtype, rows, d_ff, k, monkeypatch):
+    gen = t.Generator(device="cuda").manual_seed(rows + d_ff + k)
+    ffn = SwiGLU(ModelConfig(d_model=k, d_ff=d_ff)).to("cuda", dtype)
+    ffn.gate_up.weight.copy_((t.randn(2 * d_ff, k, generator=gen, device="cuda") * 3 / k ** 0.5).to(dtype))
+    x = t.randn(rows, k + 8, generator=gen, device="cuda").to(dtype)[:, :k]
+    gate_up = row_linear(x, ffn.gate_up.weight)
+    seen = []
+    ffn.down = t.nn.Identity()
+    handle = ffn.gate_up.register_forward_hook(lambda *a: seen.append(a[2]))
+    hooked = ffn(x)                                          # a hook sees the projection's output
+    assert len(seen) == 1 and t.equal(seen[0], gate_up) and t.equal(hooked, silu_mul(gate_up, d_ff))
+    handle.remove()
+    monkeypatch.setattr(transformer, "silu_mul", None)       # the gated kernel, nothing else
+    assert t.equal(ffn(x), hooked)
