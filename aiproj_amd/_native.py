@@ -59,6 +59,8 @@ SIGNATURES = {
     "kvfp8_rope_inplace": (_INT, [_P, _INT, _I64, _I32, _I32, _I64, _I64, _P, _INT, _P, _P, _INT, _I64, _P]),
     "kvfp8_rope_split": (_INT, [_P, _INT, _I64, _I32, _I32, _I32, _I64, _P, _INT, _P, _P, _INT, _I64, _P, _P, _P, _P]),
     "kvfp8_skinny_linear": (_INT, [_P, _INT, _I64, _I32, _I32, _P, _I64, _I32, _P, _I64, _P]),
+    "kvfp8_skinny_linear_rope": (_INT, [_P, _INT, _I64, _I32, _I32, _P, _I64, _I32, _I32, _I32, _P, _INT, _P, _P, _INT,
+                                        _I64, _P, _I64, _P]),
     "kvfp8_skinny_linear_swiglu": (_INT, [_P, _INT, _I64, _I32, _I32, _P, _I64, _I32, _P, _I64, _P]),
     "kvfp8_silu_mul": (_INT, [_P, _INT, _I64, _I32, _I64, _P, _I64, _P]),
     "kvfp8_prefill_attention": (_INT, [_P, _P, _P, _INT, _I64, _I32, _I32, _I32, _P, _INT, _I32, _I32,

@@ -173,6 +173,21 @@ struct RowDivider {
     KVFP8_HD float divide(float x) const { return fast ? corrected(x) : x / scale; }
 };
 
+// x rounded to dtype DT.
+template <int DT>
+__device__ __forceinline__ float rnd(float x) { return Elem<DT>::load(Elem<DT>::store(x)); }
+
+// One pair of the rotary embedding in place: separate multiplies and adds, every one rounded to
+// dtype DT, like the reference's elementwise operations.
+template <int DT>
+__device__ __forceinline__ void rotate_pair(float c, float s, float& x0, float& x1) {
+#pragma clang fp contract(off)
+    const float y0 = rnd<DT>(rnd<DT>(c * x0) - rnd<DT>(s * x1));
+    const float y1 = rnd<DT>(rnd<DT>(s * x0) + rnd<DT>(c * x1));
+    x0 = y0;
+    x1 = y1;
+}
+
 // silu(gate) * up.
 __device__ __forceinline__ float swiglu(float g, float u) {
     const float s = 1.0f / (1.0f + expf(-g));

@@ -27,14 +27,9 @@ struct RopeArgs {
     int64_t table_rows;
 };
 
-template <int DT>
-__device__ __forceinline__ float rnd(float x) { return Elem<DT>::load(Elem<DT>::store(x)); }
-
 template <int DT, int TT>
 __global__ void __launch_bounds__(kRopeThreads)
 rope_kernel(RopeArgs a) {
-    // Separate multiplies and adds, like the reference's elementwise operations.
-#pragma clang fp contract(off)
     using T = typename Elem<DT>::T;
     const int half = a.head_dim / 2;
     const int64_t pairs_per_row = (int64_t)a.heads * half;
@@ -52,11 +47,10 @@ rope_kernel(RopeArgs a) {
         const float c = rnd<DT>(Elem<TT>::load(reinterpret_cast<const TabT*>(a.cos_table)[pos * half + i]));
         const float s = rnd<DT>(Elem<TT>::load(reinterpret_cast<const TabT*>(a.sin_table)[pos * half + i]));
         T* e = reinterpret_cast<T*>(a.x) + r * a.row_stride + (int64_t)h * a.head_stride + 2 * i;
-        const float x0 = Elem<DT>::load(e[0]), x1 = Elem<DT>::load(e[1]);
-        const float y0 = rnd<DT>(rnd<DT>(c * x0) - rnd<DT>(s * x1));
-        const float y1 = rnd<DT>(rnd<DT>(s * x0) + rnd<DT>(c * x1));
-        e[0] = Elem<DT>::store(y0);
-        e[1] = Elem<DT>::store(y1);
+        float x0 = Elem<DT>::load(e[0]), x1 = Elem<DT>::load(e[1]);
+        rotate_pair<DT>(c, s, x0, x1);
+        e[0] = Elem<DT>::store(x0);
+        e[1] = Elem<DT>::store(x1);
     }
 }
 
@@ -76,7 +70,6 @@ struct RopeOut {
 template <int DT, int TT, bool kSplit>
 __global__ void __launch_bounds__(kRopeThreads)
 rope_vec_kernel(RopeArgs a, RopeOut out) {
-#pragma clang fp contract(off)
     using T = typename Elem<DT>::T;
     using TabT = typename Elem<TT>::T;
     struct alignas(16) Vec { T e[8]; };
@@ -101,9 +94,10 @@ rope_vec_kernel(RopeArgs a, RopeOut out) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const float cs = rnd<DT>(Elem<TT>::load(ct.e[i])), sn = rnd<DT>(Elem<TT>::load(st.e[i]));
-                const float x0 = Elem<DT>::load(v.e[2 * i]), x1 = Elem<DT>::load(v.e[2 * i + 1]);
-                v.e[2 * i] = Elem<DT>::store(rnd<DT>(rnd<DT>(cs * x0) - rnd<DT>(sn * x1)));
-                v.e[2 * i + 1] = Elem<DT>::store(rnd<DT>(rnd<DT>(sn * x0) + rnd<DT>(cs * x1)));
+                float x0 = Elem<DT>::load(v.e[2 * i]), x1 = Elem<DT>::load(v.e[2 * i + 1]);
+                rotate_pair<DT>(cs, sn, x0, x1);
+                v.e[2 * i] = Elem<DT>::store(x0);
+                v.e[2 * i + 1] = Elem<DT>::store(x1);
             }
         }
         T* dst = src;

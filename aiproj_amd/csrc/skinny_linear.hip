@@ -27,6 +27,13 @@
 // as the projection's store rounds them: the same bits as the two launches.
 // Measured (us, bf16, the two launches -> this one; the projection alone costs the same within
 // 0.6): 2 x 5632 x 2048, 64 rows 18.6 -> 15.6, 1 row 14.3 -> 11.1; 2 x 512 x 256, 64 rows 5.0 -> 2.7.
+//
+// kRotates: W is the fused q, k and v projection of a decode step and the q and k columns are
+// rotated by their row's position, in the epilogue's pairs; the projection's rounding is kept
+// here too. A thread's row is the same for every tile: its position is read once, the tile's
+// angles while the tile streams in.
+// Measured (us, bf16, the two launches -> this one, in brackets the projection alone): 3072 x
+// 2048, 64 rows 11.4 -> 8.4 [7.8], 1 row 8.4 -> 6.2 [5.4]; 768 x 256, 64 rows 5.4 -> 3.1 [2.4].
 #include "mfma_tiles.h"
 
 namespace kvfp8 {
@@ -46,7 +53,22 @@ struct LinArgs {
     int32_t groups;                          // ceil(steps / (8 waves x steps per wave))
     int32_t walkers;                         // workgroups that walk the tiles side by side
     int32_t half;                            // kGated: rows of gate, and of up
+    // kRotates: columns before `rotated` turn by the angles of positions[row] in the tables
+    // [table_rows][head_dim / 2] (rows of positions outside them stay).
+    const void* positions;
+    const void* cos_table;
+    const void* sin_table;
+    int64_t table_rows;
+    int32_t pos64, table_dtype, rotated, head_dim;
 };
+
+enum { kPlain, kGate, kRotate };             // what the epilogue does
+
+__device__ __forceinline__ float table_value(const void* table, int dtype, int64_t at) {
+    if (dtype == KVFP8_F32) return reinterpret_cast<const float*>(table)[at];
+    const uint16_t x = reinterpret_cast<const uint16_t*>(table)[at];
+    return dtype == KVFP8_F16 ? Elem<KVFP8_F16>::load(x) : Elem<KVFP8_BF16>::load(x);
+}
 
 // Barrier over LDS accesses only: __syncthreads would also wait for the block in flight.
 __device__ __forceinline__ void lds_barrier() {
@@ -55,9 +77,10 @@ __device__ __forceinline__ void lds_barrier() {
     __asm__ volatile("" ::: "memory");
 }
 
-template <int MT, int STEPS, bool kF16, bool kGated>
+template <int MT, int STEPS, bool kF16, int kEpi>
 __global__ void __launch_bounds__(64 * kLinWaves, 2)
 skinny_linear_kernel(LinArgs a) {
+    constexpr bool kGated = kEpi == kGate, kRotates = kEpi == kRotate;
     constexpr int ROW = STEPS * 64;                  // bytes of a row's slice
     constexpr int CPR = ROW / 16;                    // 16-byte chunks of it
     constexpr int MASK = CPR < 16 ? CPR - 1 : 15;    // chunk c of row r sits in slot c ^ (r & MASK)
@@ -128,11 +151,37 @@ skinny_linear_kernel(LinArgs a) {
         __asm__ volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     };
 
+    // The epilogue's thread: two neighbouring outputs (col, col + 1 of the tile) of one row of x.
+    using E = Elem<kF16 ? KVFP8_F16 : KVFP8_BF16>;
+    constexpr int kCols = kGated ? kLinRows / 2 : kLinRows;
+    constexpr int kPairs = MT * 16 * kCols / 2;
+    const int local = 2 * (int)threadIdx.x / kCols, col = 2 * (int)threadIdx.x % kCols, row = m0 + local;
+    const bool stores = (int)threadIdx.x < kPairs && row < a.rows;
+
     u32x4_t x[MT][STEPS];
     f32x4_t acc[MT];
     int slot = 0;
     load_next();
+    int64_t pos = -1;
+    if constexpr (kRotates) {
+        if (stores)
+            pos = a.pos64 ? reinterpret_cast<const int64_t*>(a.positions)[row]
+                          : (int64_t)reinterpret_cast<const int32_t*>(a.positions)[row];
+        // Arrived before the loop, where a wait for it would wait for the block in flight too.
+        __asm__ volatile("" : "+v"(pos));
+    }
     for (int tile = first; tile < a.tiles; tile += a.walkers) {
+        float cs = 1.0f, sn = 0.0f;
+        bool turn = false;
+        if constexpr (kRotates) {
+            const int at = tile * kLinRows + col;
+            turn = at < a.rotated && pos >= 0 && pos < a.table_rows;
+            if (turn) {
+                const int64_t angle = pos * (a.head_dim / 2) + (at % a.head_dim) / 2;
+                cs = table_value(a.cos_table, a.table_dtype, angle);
+                sn = table_value(a.sin_table, a.table_dtype, angle);
+            }
+        }
         for (int group = 0; group < a.groups; ++group) {
             if (a.groups > 1 || tile == first) {
 #pragma unroll
@@ -175,14 +224,9 @@ skinny_linear_kernel(LinArgs a) {
             }
             return sum;
         };
-        // Thread: two neighbouring outputs of one row of x.
-        constexpr int kCols = kGated ? kLinRows / 2 : kLinRows;
-        constexpr int kPairs = MT * 16 * kCols / 2;
-        if ((int)threadIdx.x < kPairs) {
-            const int local = 2 * threadIdx.x / kCols, col = 2 * threadIdx.x % kCols, row = m0 + local;
+        if (stores) {
             uint32_t out;
             if constexpr (kGated) {
-                using E = Elem<kF16 ? KVFP8_F16 : KVFP8_BF16>;
                 const float2 gate = sum2(local * kLinRows + col), up = sum2(local * kLinRows + 8 + col);
                 const uint32_t g = pack2<kF16>(gate.x, gate.y), u = pack2<kF16>(up.x, up.y);
                 out = pack2<kF16>(swiglu(E::load((uint16_t)g), E::load((uint16_t)u)),
@@ -190,9 +234,16 @@ skinny_linear_kernel(LinArgs a) {
             } else {
                 const float2 sum = sum2(local * kLinRows + col);
                 out = pack2<kF16>(sum.x, sum.y);
+                if constexpr (kRotates) {
+                    constexpr int DT = kF16 ? KVFP8_F16 : KVFP8_BF16;
+                    if (turn) {
+                        float x0 = E::load((uint16_t)out), x1 = E::load((uint16_t)(out >> 16));
+                        rotate_pair<DT>(rnd<DT>(cs), rnd<DT>(sn), x0, x1);
+                        out = pack2<kF16>(x0, x1);
+                    }
+                }
             }
-            if (row < a.rows)
-                *reinterpret_cast<uint32_t*>(a.y + row * a.y_row + (int64_t)(tile * kCols + col) * 2) = out;
+            *reinterpret_cast<uint32_t*>(a.y + row * a.y_row + (int64_t)(tile * kCols + col) * 2) = out;
         }
         lds_barrier();
     }
@@ -214,11 +265,14 @@ template <int MT, int STEPS>
 hipError_t launch_linear(const LinArgs& a, bool f16, int grid, hipStream_t s) {
     const dim3 g(grid), b(64 * kLinWaves);
     if (a.half > 0) {
-        if (f16) hipLaunchKernelGGL((skinny_linear_kernel<MT, STEPS, true, true>), g, b, 0, s, a);
-        else hipLaunchKernelGGL((skinny_linear_kernel<MT, STEPS, false, true>), g, b, 0, s, a);
+        if (f16) hipLaunchKernelGGL((skinny_linear_kernel<MT, STEPS, true, kGate>), g, b, 0, s, a);
+        else hipLaunchKernelGGL((skinny_linear_kernel<MT, STEPS, false, kGate>), g, b, 0, s, a);
+    } else if (a.rotated > 0) {
+        if (f16) hipLaunchKernelGGL((skinny_linear_kernel<MT, STEPS, true, kRotate>), g, b, 0, s, a);
+        else hipLaunchKernelGGL((skinny_linear_kernel<MT, STEPS, false, kRotate>), g, b, 0, s, a);
     } else {
-        if (f16) hipLaunchKernelGGL((skinny_linear_kernel<MT, STEPS, true, false>), g, b, 0, s, a);
-        else hipLaunchKernelGGL((skinny_linear_kernel<MT, STEPS, false, false>), g, b, 0, s, a);
+        if (f16) hipLaunchKernelGGL((skinny_linear_kernel<MT, STEPS, true, kPlain>), g, b, 0, s, a);
+        else hipLaunchKernelGGL((skinny_linear_kernel<MT, STEPS, false, kPlain>), g, b, 0, s, a);
     }
     return hipGetLastError();
 }
@@ -240,9 +294,9 @@ using namespace kvfp8;
 
 namespace {
 
-// n: weight rows; half: 0, or n / 2 for a gated output of that many columns.
-int skinny_linear(const void* x, int dtype, int64_t x_stride, int32_t rows, int32_t k, const void* weight,
-                  int64_t w_stride, int32_t n, int32_t half, void* out, int64_t out_stride, void* stream) {
+// n: weight rows; a: what the epilogue needs (zeros for plain).
+int skinny_linear(LinArgs a, const void* x, int dtype, int64_t x_stride, int32_t rows, int32_t k, const void* weight,
+                  int64_t w_stride, int32_t n, void* out, int64_t out_stride, void* stream) {
     if (dtype != KVFP8_BF16 && dtype != KVFP8_F16) return KVFP8_EDTYPE;
     if (rows < 0 || rows > 64 || k <= 0 || k % 32 != 0 || n <= 0 || n % kLinRows != 0) return KVFP8_ESHAPE;
     if (rows == 0) return KVFP8_OK;
@@ -250,7 +304,6 @@ int skinny_linear(const void* x, int dtype, int64_t x_stride, int32_t rows, int3
     if ((((uintptr_t)x | (uintptr_t)weight) & 15) != 0 || ((uintptr_t)out & 3) != 0 || x_stride % 8 != 0 ||
         w_stride % 8 != 0 || out_stride % 2 != 0 || w_stride < k)
         return KVFP8_ESTRIDE;
-    LinArgs a;
     a.x = reinterpret_cast<const uint8_t*>(x);
     a.w = reinterpret_cast<const uint8_t*>(weight);
     a.y = reinterpret_cast<uint8_t*>(out);
@@ -259,7 +312,6 @@ int skinny_linear(const void* x, int dtype, int64_t x_stride, int32_t rows, int3
     a.y_row = out_stride * 2;
     a.rows = rows;
     a.tiles = n / kLinRows;
-    a.half = half;
     a.steps = k / 32;
     int per_wave = 2;
     while (per_wave < kLinSteps && kLinWaves * per_wave < a.steps) per_wave *= 2;
@@ -288,12 +340,36 @@ int skinny_linear(const void* x, int dtype, int64_t x_stride, int32_t rows, int3
 extern "C" int kvfp8_skinny_linear(const void* x, int dtype, int64_t x_stride, int32_t rows, int32_t k,
                                    const void* weight, int64_t w_stride, int32_t n, void* out, int64_t out_stride,
                                    void* stream) {
-    return skinny_linear(x, dtype, x_stride, rows, k, weight, w_stride, n, 0, out, out_stride, stream);
+    return skinny_linear(LinArgs{}, x, dtype, x_stride, rows, k, weight, w_stride, n, out, out_stride, stream);
 }
 
 extern "C" int kvfp8_skinny_linear_swiglu(const void* x, int dtype, int64_t x_stride, int32_t rows, int32_t k,
                                           const void* weight, int64_t w_stride, int32_t n, void* out,
                                           int64_t out_stride, void* stream) {
     if (n <= 0 || n % (kLinRows / 2) != 0 || n > (1 << 30)) return KVFP8_ESHAPE;
-    return skinny_linear(x, dtype, x_stride, rows, k, weight, w_stride, 2 * n, n, out, out_stride, stream);
+    LinArgs a{};
+    a.half = n;
+    return skinny_linear(a, x, dtype, x_stride, rows, k, weight, w_stride, 2 * n, out, out_stride, stream);
+}
+
+extern "C" int kvfp8_skinny_linear_rope(const void* x, int dtype, int64_t x_stride, int32_t rows, int32_t k,
+                                        const void* weight, int64_t w_stride, int32_t n, int32_t heads,
+                                        int32_t head_dim, const void* positions, int pos_dtype, const void* cos_table,
+                                        const void* sin_table, int table_dtype, int64_t table_rows, void* out,
+                                        int64_t out_stride, void* stream) {
+    if (table_dtype != KVFP8_F32 && table_dtype != KVFP8_F16 && table_dtype != KVFP8_BF16) return KVFP8_EDTYPE;
+    if (pos_dtype != KVFP8_I32 && pos_dtype != KVFP8_I64) return KVFP8_EDTYPE;
+    if (heads <= 0 || head_dim <= 0 || head_dim % 2 != 0 || table_rows <= 0 || (int64_t)heads * head_dim > n)
+        return KVFP8_ESHAPE;
+    if (rows > 0 && (!positions || !cos_table || !sin_table)) return KVFP8_ENULL;
+    LinArgs a{};
+    a.positions = positions;
+    a.pos64 = pos_dtype == KVFP8_I64;
+    a.cos_table = cos_table;
+    a.sin_table = sin_table;
+    a.table_dtype = table_dtype;
+    a.table_rows = table_rows;
+    a.rotated = heads * head_dim;
+    a.head_dim = head_dim;
+    return skinny_linear(a, x, dtype, x_stride, rows, k, weight, w_stride, n, out, out_stride, stream);
 }

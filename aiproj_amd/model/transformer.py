@@ -23,7 +23,7 @@ norm), RoPE, the SwiGLU activation, the cache write and the decode attention are
 library's HIP kernels (in decode, the new token's quantized write is done by the decode
 kernel itself);
 the projections and the FFN are `RowLinear`: the HIP kernel `skinny_linear_kernel` for the
-few rows of a decode step, plain GEMMs (hipBLASLt through torch) otherwise; prompt
+few rows of a decode step, which then also does RoPE and the activation, plain GEMMs (hipBLASLt through torch) otherwise; prompt
 (prefill) attention is the varlen causal HIP kernel behind `flash_attention_forward`,
 as the reference calls its FlashAttentionFunction there (`attention.py:103-110`).
 """
@@ -104,6 +104,17 @@ class RoPE(nn.Module):
         _native.check(rc, "kvfp8_rope_inplace")
         return x
 
+    def project(self, x: t.Tensor, weight: t.Tensor, positions: t.Tensor, heads: int) -> t.Tensor:
+        """`apply_` of x weight^T, one launch (rows and weights that `_takes_skinny` names)."""
+        from aiproj_amd import _native
+
+        _native.require_gpu(x, positions, what="rope")
+        if not self.cos_table.is_contiguous():
+            raise ValueError("rope: rows need unit element stride")
+        return _skinny("kvfp8_skinny_linear_rope", x, weight, weight.shape[0], heads, self.head_dim,
+                       positions.data_ptr(), _native.dtype_code(positions.dtype), self.cos_table.data_ptr(),
+                       self.sin_table.data_ptr(), _native.dtype_code(self.cos_table.dtype), self.cos_table.shape[0])
+
     def split(self, qkv: t.Tensor, positions: t.Tensor, num_q_heads: int, num_kv_heads: int):
         """Packed q and k (rotated) and v of fused projection rows [q heads | k heads | v heads],
         one launch of `rope_vec_kernel`; None for rows it does not take."""
@@ -144,12 +155,12 @@ def _takes_skinny(x: t.Tensor, weight: t.Tensor) -> bool:
                 or not _native.is_plain(x, weight) or x.data_ptr() % 16 or weight.data_ptr() % 16)
 
 
-def _skinny(entry: str, x: t.Tensor, weight: t.Tensor, columns: int) -> t.Tensor:
+def _skinny(entry: str, x: t.Tensor, weight: t.Tensor, columns: int, *more) -> t.Tensor:
     from aiproj_amd import _native
 
     out = t.empty((x.shape[0], columns), dtype=x.dtype, device=x.device)
     rc = getattr(_native.lib(), entry)(x.data_ptr(), _native.dtype_code(x.dtype), x.stride(0), x.shape[0], x.shape[1],
-                                       weight.data_ptr(), weight.stride(0), columns, out.data_ptr(), columns,
+                                       weight.data_ptr(), weight.stride(0), columns, *more, out.data_ptr(), columns,
                                        _native.stream_handle(x.device))
     _native.check(rc, entry)
     return out
@@ -192,8 +203,14 @@ class Attention(nn.Module):
 
     def forward(self, h: t.Tensor, meta: StepMeta, cache) -> t.Tensor:
         cfg = self.cfg
-        qkv = self.qkv_proj(h)
         ctx = meta.cache_context
+        proj = self.qkv_proj
+        # A decode step's rotation is done by the projection's kernel (`kvfp8_skinny_linear_rope`).
+        if (meta.mode != "prefill" and isinstance(proj, RowLinear) and proj.unobserved() and type(self.rope) is RoPE
+                and proj.weight.shape[0] == self.q_dim + 2 * self.kv_dim and _takes_skinny(h, proj.weight)):
+            qkv = self.rope.project(h, proj.weight, meta.token_positions, cfg.num_q_heads + cfg.num_kv_heads)
+            return self._attend(qkv, meta, cache)
+        qkv = proj(h)
         if meta.mode == "prefill":
             # Prompt attention takes packed q, k and v: rotated and split in one pass.
             split = self.rope.split(qkv, meta.token_positions, cfg.num_q_heads, cfg.num_kv_heads)
@@ -204,6 +221,11 @@ class Attention(nn.Module):
                 return self.o_proj(out.reshape(-1, self.q_dim))
         # q and k heads are the first Hq + Hkv heads of every row: one in-place rotation.
         self.rope.apply_(qkv, meta.token_positions, cfg.num_q_heads + cfg.num_kv_heads)
+        return self._attend(qkv, meta, cache)
+
+    def _attend(self, qkv: t.Tensor, meta: StepMeta, cache) -> t.Tensor:
+        """The cache write, the attention and the output projection of rotated fused rows."""
+        cfg, ctx = self.cfg, meta.cache_context
         q = qkv[:, :self.q_dim].view(-1, cfg.num_q_heads, cfg.head_dim)
         k = qkv[:, self.q_dim:self.q_dim + self.kv_dim].view(-1, cfg.num_kv_heads, cfg.head_dim)
         v = qkv[:, self.q_dim + self.kv_dim:].view(-1, cfg.num_kv_heads, cfg.head_dim)

@@ -387,6 +387,17 @@ int kvfp8_skinny_linear_swiglu(const void* x_dev, int dtype, int64_t x_stride, i
                                const void* weight_dev, int64_t w_stride, int32_t n, void* out_dev,
                                int64_t out_stride, void* stream);
 
+/*
+ * kvfp8_skinny_linear followed by kvfp8_rope_inplace over the first `heads` heads of head_dim
+ * columns, bit for bit, in one launch. heads * head_dim at most n; positions, tables and rows
+ * outside them as kvfp8_rope_inplace.
+ */
+int kvfp8_skinny_linear_rope(const void* x_dev, int dtype, int64_t x_stride, int32_t rows, int32_t k,
+                             const void* weight_dev, int64_t w_stride, int32_t n, int32_t heads, int32_t head_dim,
+                             const void* positions_dev, int pos_dtype, const void* cos_table_dev,
+                             const void* sin_table_dev, int table_dtype, int64_t table_rows, void* out_dev,
+                             int64_t out_stride, void* stream);
+
 /* Human-readable name of a return code (negative KVFP8_E* or positive hipError_t). */
 const char* kvfp8_strerror(int code);
 

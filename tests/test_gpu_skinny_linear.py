@@ -5,7 +5,7 @@ import pytest
 import torch as t
 
 from aiproj_amd.model import transformer
-from aiproj_amd.model.transformer import ModelConfig, RowLinear, SwiGLU, row_linear, silu_mul
+from aiproj_amd.model.transformer import ModelConfig, RoPE, RowLinear, SwiGLU, row_linear, silu_mul
 
 pytestmark = pytest.mark.gpu
 
@@ -75,3 +75,20 @@ def test_gated_projection_equals_the_two_launches(dtype, rows, d_ff, k, monkeypa
     handle.remove()
     monkeypatch.setattr(transformer, "silu_mul", None)       # the gated kernel, nothing else
     assert t.equal(ffn(x), hooked)
+
+
+# Head sizes of one and several tiles, ends of the rotated columns inside a tile, both position
+# types, positions outside the tables, rows divided over workgroups, several tiles per workgroup.
+@t.no_grad()
+@pytest.mark.parametrize("dtype,table", [(t.bfloat16, t.bfloat16), (t.float16, t.float32), (t.bfloat16, t.float16)])
+@pytest.mark.parametrize("rows", [1, 17, 33, 64])
+@pytest.mark.parametrize("heads,d,n,k", [(1, 16, 32, 32), (3, 8, 48, 96), (5, 20, 112, 1024), (20, 128, 3072, 2048),
+                                         (40, 128, 6144, 288)])
+def test_rotated_projection_equals_the_two_launches(dtype, table, rows, heads, d, n, k):
+    gen = t.Generator(device="cuda").manual_seed(rows + n + k)
+    w = (t.randn(n, k, generator=gen, device="cuda") / k ** 0.5).to(dtype)
+    x = t.randn(rows, k + 8, generator=gen, device="cuda").to(dtype)[:, :k]
+    rope = RoPE(d, 96, 10000.0).to("cuda", table)
+    pos = t.randint(-2, 98, (rows,), generator=gen, device="cuda", dtype=t.int32 if rows % 2 else t.int64)
+    want = rope.apply_(row_linear(x, w), pos, heads)
+    assert t.equal(rope.project(x, w, pos, heads), want)
