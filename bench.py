@@ -479,7 +479,7 @@ def kernel_legs(steps: int):
       * f16 (with f16 q, on the MFMA kernel) and f32 (grouped VALU kernel) caches at the
         north-star shape;
       * MFMA against the grouped VALU kernel on the same FP8 bytes (north, cfg4);
-      * the grouped kernel at head size 80, a shape the MFMA kernel does not take."""
+      * head size 80, the MFMA kernel's narrow rows."""
     import torch as t
     import oracle
     from aiproj_amd import workloads
@@ -552,8 +552,8 @@ def kernel_legs(steps: int):
         w = workloads.build(spec, "cuda")
         caches = pools_for(w, t.float8_e4m3fn, spec)
         split_us, call_us = _time_decode(caches, w.q, workloads.make_context(w), max(4, steps // 4))
-        legs["fp8_d80_valu"] = entry(spec, 1, split_us, call_us, "decode_split_grouped + decode_combine (D 80)")
-        log(f"[grouped D80] split {split_us:.1f} us, split + combine {call_us:.1f} us")
+        legs["fp8_d80"] = entry(spec, 1, split_us, call_us, "decode_mfma_kernel + combine_mfma_kernel (D 80)")
+        log(f"[D80] split {split_us:.1f} us, split + combine {call_us:.1f} us")
         del caches
         t.cuda.empty_cache()
     return legs
