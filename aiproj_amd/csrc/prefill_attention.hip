@@ -434,8 +434,13 @@ prefill_attention_kernel(PrefillArgs a) {
 // Head sizes between 64 and 128 keep the LDS rows of 128 (16 chunk slots of 16 bytes, the
 // swizzle needs a power of two) and load only their own chunks; the products run over
 // exactly D: 32-dim steps and, for an odd multiple of 16, one 16-dim step (MFMA 16x16x16).
-// Measured, 16 prompts of 64 to 1984 tokens, 32q/8kv heads, D 80, f16: 1024 us on the
-// general kernel above (which pads every product to 128 dims) -> 452 us.
+// They keep the general kernel's precision: their reference maximum moves with every row's
+// maximum. Behind it by up to 2^8, as for 64 and 128, the largest probability is rounded to
+// 16 bits while the denominator is not: error against 64 bits 2.47e-4 -> 2.53e-4 for flat
+// rows and 2.16e-4 -> 2.54e-4 for peaked ones (f16, D 80).
+// Measured, 16 prompts of 64 to 1984 tokens, 32q/8kv heads, D 80, f16: 1127 us on the
+// general kernel above (which pads every product to 128 dims) -> 443 us; in another order of
+// the lengths 483 us, and 440 us with the reference of 64 and 128.
 //
 // An item is one (sequence, KV head, query block): the eight waves are `gw` q heads
 // x (8 / gw) groups of 32 query rows, and its K/V blocks of 64 keys are staged once
@@ -533,6 +538,10 @@ prefill_fa_kernel(PrefillArgs a, int32_t units, int32_t upx, int32_t per_xcd) {
     constexpr int NB = kD / 16;                      // 16-dim tiles of the PV product
     constexpr int KS = kD / 32;                      // 32-dim steps of the QK product
     constexpr bool kHalf = kD % 32 != 0;             // and one step of 16 dims
+    // How far (log2) a row's max may exceed the reference that its probabilities are scaled by.
+    // 80, 96 and 112: not at all, so that the largest probability is 1 and packed without error,
+    // as on the general kernel (see above).
+    constexpr float kLag = kD == 64 || kD == 128 ? 8.0f : 0.0f;
     // Vector-memory instructions a wave issues: kBlockLoads per K/V block, kQLoads
     // for its Q operands of one item.
     constexpr int kBlockLoads = 2 * CPT;
@@ -810,12 +819,12 @@ prefill_fa_kernel(PrefillArgs a, int32_t units, int32_t upx, int32_t per_xcd) {
 #pragma unroll
             for (int i = 1; i < 16; ++i) mx = fmaxf(mx, sacc[i / 4][qt][i % 4]);
             mx *= a.scale_log2;                        // base-2 units (scale > 0 keeps the order)
-            // Lazy rescale: the accumulators keep a reference max m that is only moved
+            // Lazy rescale (kLag): the accumulators keep a reference max m that is only moved
             // when some row's max grows by more than 2^8 (p <= 256 meanwhile, far
             // inside float32 and bf16 range), so the accumulators are rarely scaled.
             // Each lane tests its own 16 keys; only a rescale needs the row's max over
             // its four lanes.
-            if (__ballot(mx > m[qt] + 8.0f)) {
+            if (__ballot(mx > m[qt] + kLag)) {
                 const float m_new = fmaxf(m[qt], max_across_rows(mx));
                 const float m_use = m_new == kNegInf ? 0.0f : m_new;
                 // An item's first block finds the accumulators at zero: nothing to scale.

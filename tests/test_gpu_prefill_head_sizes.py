@@ -32,3 +32,24 @@ def test_wide_kernel_head_sizes(dtype, head_dim, sign):
     tol = TOLERANCE[dtype]
     t.testing.assert_close(out.double().cpu(), t.from_numpy(want), rtol=tol, atol=tol)
     t.testing.assert_close(lse.double().cpu(), t.from_numpy(want_lse), rtol=1e-3, atol=1e-3)
+
+
+@t.inference_mode()
+@pytest.mark.parametrize("dtype,half_ulp", [(t.float16, 2.0 ** -11), (t.bfloat16, 2.0 ** -8)])
+@pytest.mark.parametrize("head_dim", [80, 96, 112])
+def test_largest_probability_is_exact(dtype, half_ulp, head_dim):
+    """The last of 65 keys exceeds the others (all 0) by up to 2^8, in a block of its own, and
+    alone has values: its probability is 1 in 16 bits, so the output has one rounding (and
+    float32 error, below 4e-6) and no second one from the probability."""
+    sequences, hq = 96, 4
+    gen = t.Generator(device="cuda").manual_seed(head_dim)
+    q, k, v = (t.zeros(65 * sequences, h, head_dim, device="cuda", dtype=dtype) for h in (hq, 1, 1))
+    last = t.arange(64, 65 * sequences, 65, device="cuda")
+    scores = 5.5 * t.rand(sequences, hq, 1, device="cuda", generator=gen)
+    q[last] = (scores / math.sqrt(head_dim)).expand(-1, -1, head_dim).to(dtype)
+    k[last] = 1
+    v[last] = (1 + t.rand(sequences, 1, head_dim, device="cuda", generator=gen)).to(dtype)
+    cu = t.arange(0, 65 * sequences + 1, 65, dtype=t.int32, device="cuda")
+    out, _ = flash_attention_forward(q, k, v, cu, 65, 1 / math.sqrt(head_dim))
+    e = t.exp(q[last].double().sum(-1, keepdim=True) / math.sqrt(head_dim))
+    t.testing.assert_close(out[last].double(), v[last].double() * (e / (64 + e)), rtol=half_ulp + 4e-6, atol=0)
