@@ -6,12 +6,16 @@
 //   dV = P^T dO,   dS = P (dP - delta),   dQ = scale dS K,   dK = scale dS^T Q,
 // dK and dV summed over the q heads of a KV head.
 //
-// Precision. Every product has float32 accuracy: the matrix cores multiply bf16 values
-// exactly and add in float32, and a float32 factor enters as the sum of three bf16
-// values (8 + 8 + 8 mantissa bits, split by truncation, so nothing is lost). bf16 inputs
-// are one such plane, float16 inputs two, float32 inputs three (`split_planes_kernel`);
-// P and dS, computed in float32, are always three. Products of planes i and j with
-// i + j > 2 lie below float32's last bit and are left out.
+// Precision. Products are those of float32: the matrix cores multiply bf16 values exactly
+// and add in float32, and a float32 factor enters as the sum of three bf16 values (`split3`:
+// nothing is lost). bf16 inputs are one such plane, float16 inputs two, float32 inputs three
+// (`split_planes_kernel`); P and dS, computed in float32, are always three. Products of planes
+// i and j with i + j > 2 are left out: none for bf16 inputs, else two of at most 2^-25 of
+// their product each (parts to nearest), of either sign.
+// Measured against 64 bits, float32 inputs, 8q/2kv heads, D 64, sequences of 40 to 700 (dk and
+// dv): PyTorch's float32 operations 4.5e-7 and 4.0e-7, this kernel 2.4e-7 and 2.2e-7; inputs
+// of one sign 2.1e-7 and 1.2e-7, this kernel 1.1e-7 and 0.8e-7 (with truncated parts 1.4e-6
+// and 4.1e-7: the products left out are then up to 2^-22, all of the sign of the product).
 //
 // Bound: instruction issue on the matrix cores and the vector ALU. Per pair of tiles with
 // bf16 inputs: one product each for S and dP in either pass, three for each gradient; the
@@ -77,17 +81,22 @@ struct BwdArgs {
     float* part;                   // their sums [dK, dV][split][T][Hkv][d] when splits > 1
 };
 
-// x as three bf16 values by truncation, hi + mid + lo = x exactly (normal x); the parts
-// of two floats share a dword. Infinite x leaves NaN parts: non-finite either way.
+// x as three bf16 values, hi + mid + lo = x exactly (normal x); the parts of two floats share
+// a dword. Truncated (kNearest false): the parts have x's sign and reach 2^-7 and 2^-15 of it,
+// for one-plane inputs, where every product is added up. To nearest: 2^-8 and 2^-17, of either
+// sign, for inputs of several planes, where some products are left out. Infinite x leaves NaN
+// parts: non-finite either way.
+template <bool kNearest>
 __device__ __forceinline__ void split3(float x0, float x1, u32x4_t (&out)[3], int dword) {
     float r0 = x0, r1 = x1;
 #pragma unroll
     for (int p = 0; p < 3; ++p) {
         const uint32_t b0 = f32_bits(r0), b1 = f32_bits(r1);
-        out[p][dword] = __builtin_amdgcn_perm(b1, b0, 0x07060302u);
+        const uint32_t two = kNearest ? pack2<false>(r0, r1) : __builtin_amdgcn_perm(b1, b0, 0x07060302u);
+        out[p][dword] = two;
         if (p < 2) {
-            r0 -= bits_f32(b0 & 0xFFFF0000u);
-            r1 -= bits_f32(b1 & 0xFFFF0000u);
+            r0 -= bits_f32(kNearest ? two << 16 : b0 & 0xFFFF0000u);
+            r1 -= bits_f32((kNearest ? two : b1) & 0xFFFF0000u);
         }
     }
 }
@@ -351,13 +360,13 @@ __device__ __forceinline__ void bwd_item(const BwdArgs& a, int64_t item, uint8_t
         u32x4_t w[3];
         if constexpr (!kDq) {
 #pragma unroll
-            for (int u = 0; u < 4; ++u) split3(pr[u / 2][2 * (u % 2)], pr[u / 2][2 * (u % 2) + 1], w, u);
+            for (int u = 0; u < 4; ++u) split3<(NP > 1)>(pr[u / 2][2 * (u % 2)], pr[u / 2][2 * (u % 2) + 1], w, u);
             gradient(1, 1, w, pp, buf_off);
         }
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
             const int h = u / 2, jj = 2 * (u % 2);
-            split3(pr[h][jj] * dp[0][h][jj], pr[h][jj + 1] * dp[0][h][jj + 1], w, u);
+            split3<(NP > 1)>(pr[h][jj] * dp[0][h][jj], pr[h][jj + 1] * dp[0][h][jj + 1], w, u);
         }
         gradient(0, 0, w, pp, buf_off);
     };
@@ -622,7 +631,9 @@ split_planes_kernel(PlaneArgs a) {
         const float x0 = d0 < a.d ? Elem<IT>::load(in[0]) : 0.0f;
         const float x1 = d0 + 1 < a.d ? Elem<IT>::load(in[1]) : 0.0f;
         u32x4_t planes[3];
-        split3(x0, x1, planes, 0);
+        // (Finite values above the largest bf16 would round to infinity.)
+        if (fmaxf(__builtin_fabsf(x0), __builtin_fabsf(x1)) > 3.3895313e38f) split3<false>(x0, x1, planes, 0);
+        else split3<true>(x0, x1, planes, 0);
         for (int p = 0; p < a.planes; ++p) a.out[t][(p * rows + row) * pairs + c] = planes[p][0];
     }
 }

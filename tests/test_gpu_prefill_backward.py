@@ -107,3 +107,29 @@ def test_unaligned_inputs_and_other_calls():
     strided = grad.transpose(0, 1).contiguous().transpose(0, 1)
     assert fa._native_backward(q, k, v, out, lse, cu, strided, 70, 0.125) is None
     check(fa.flash_attention_backward(q, k, v, out, lse, cu, strided, 70, 0.125), want, t.bfloat16)
+
+
+@pytest.mark.parametrize("d", [64, 80, 128])
+@pytest.mark.parametrize("positive", [False, True])
+def test_float32_is_no_less_exact_than_torch(d, positive):
+    """Against 64 bits, from the exact output and lse: the error of the float32 gradients is at most
+    that of PyTorch's float32 operations (twice as large here would be a lost bit), also where all
+    terms of the sums have one sign, which one-sided errors of the products would not survive."""
+    lengths = [40, 100, 300, 700]
+    bounds, rows = inputs(lengths, 8, 2, d, t.float32, seed=d)
+    q, k, v, grad = (x.abs() + 0.5 if positive else x for x in rows)
+    cu = t.tensor(bounds, dtype=t.int32, device="cuda")
+    scale = 1 / math.sqrt(d)
+    out, lse = t.empty(q.shape, dtype=t.float64, device="cuda"), t.empty(q.shape[:2], dtype=t.float64, device="cuda")
+    for s0, s1 in zip(bounds, bounds[1:]):
+        qs, ks, vs = (x[s0:s1].double().transpose(0, 1) for x in (q, k, v))
+        ks, vs = ks.repeat_interleave(4, 0), vs.repeat_interleave(4, 0)
+        s = t.matmul(qs, ks.transpose(1, 2).contiguous()) * scale
+        s = s.masked_fill(t.ones(s.shape[1:], dtype=t.bool, device="cuda").triu(1), -math.inf)
+        out[s0:s1], lse[s0:s1] = t.matmul(t.softmax(s, -1), vs).transpose(0, 1), t.logsumexp(s, -1).T
+    out, lse = out.float(), lse.float()
+    got = fa._native_backward(q, k, v, out, lse, cu, grad, max(lengths), scale)
+    strided = grad.transpose(0, 1).contiguous().transpose(0, 1)
+    torch_got = fa.flash_attention_backward(q, k, v, out, lse, cu, strided, max(lengths), scale)
+    for g, x, w in zip(got, torch_got, reference(q, k, v, bounds, max(lengths), grad)):
+        assert float((g.double() - w).norm()) <= 1.1 * float((x.double() - w).norm())
