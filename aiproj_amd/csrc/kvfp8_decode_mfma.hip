@@ -442,6 +442,12 @@ __device__ __forceinline__ void compute_step(WaveState<C>& st, const StepData<C,
     const bool full = lim_a == 16 && lim_b == 16;   // wave-uniform
 
     constexpr bool kWL = kWholeRowK<C, ES, kNarrow>;
+    // float32 q on narrow rows: the products of lower parts are summed on their own, so that the
+    // large sums are rounded no more often than on the vector ALU. Error against float64 (q of
+    // deviation 4, D 80): vector ALU 2.9e-7, all parts in one chain 4.4e-7, this 2.3e-7. Time
+    // (B 32 x 2000, 32q/8kv, D 80; B 64, 16q/4kv, D 96): vector ALU 39.4 and 235 us, one chain
+    // 33.6 and 34.6, this 35.0 and 38.7.
+    constexpr bool kExactQ = kNarrow && kQP == 3;
     // Per-token scales of score i (k, with sm_scale * log2(e)) and V row i (v).
     float ks[8], vs[8];
     if constexpr (ES == 1) {
@@ -521,7 +527,7 @@ __device__ __forceinline__ void compute_step(WaveState<C>& st, const StepData<C,
             }
         }
     } else {
-        f32x4_t sa = {0.0f, 0.0f, 0.0f, 0.0f}, sb = {0.0f, 0.0f, 0.0f, 0.0f};
+        f32x4_t sa = {0.0f, 0.0f, 0.0f, 0.0f}, sb = sa, sa_lo = sa, sb_lo = sa;
 #pragma unroll
         for (int kb = 0; kb < 2 * C; ++kb) {
             Op ka, kbv;
@@ -535,9 +541,15 @@ __device__ __forceinline__ void compute_step(WaveState<C>& st, const StepData<C,
             }
 #pragma unroll
             for (int p = 0; p < kQP; ++p) {
-                sa = mma(ka, q[p][kb], sa);
-                sb = mma(kbv, q[p][kb], sb);
+                f32x4_t& da = kExactQ && p > 0 ? sa_lo : sa;
+                f32x4_t& db = kExactQ && p > 0 ? sb_lo : sb;
+                da = mma(ka, q[p][kb], da);
+                db = mma(kbv, q[p][kb], db);
             }
+        }
+        if constexpr (kExactQ) {
+            sa += sa_lo;
+            sb += sb_lo;
         }
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -617,6 +629,13 @@ __device__ __forceinline__ void compute_step(WaveState<C>& st, const StepData<C,
 #pragma unroll
             for (int x = 0; x < 4; ++x) {
                 const bf16x8_t av = cat8(e[x][0], e[x][1], e[x][2], e[x][3]);
+                if constexpr (kExactQ) {
+                    f32x4_t sum = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                    for (int p = kPP - 1; p >= 0; --p) sum = mma(av, pp[p], sum);
+                    st.o[4 * c + x] += sum;
+                    continue;
+                }
 #pragma unroll
                 for (int p = 0; p < kPP; ++p) st.o[4 * c + x] = mma(av, pp[p], st.o[4 * c + x]);
             }

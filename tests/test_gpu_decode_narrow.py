@@ -78,6 +78,30 @@ def test_narrow_heads_match_float64(q_dtype, cache_dtype, hq, hkv, d):
     assert float((out.double() - want).norm()) <= TOLERANCE[q_dtype] * float(want.norm())
 
 
+@pytest.mark.parametrize("d", [80, 96, 112])
+@pytest.mark.parametrize("sharp", [1, 4])
+def test_float32_q_is_no_less_exact_than_the_vector_alu(d, sharp):
+    """The error against float64 is at most that of the vector-ALU kernels, which take the same bytes
+    off a 16-byte boundary (the margin is the spread of two orders of float32 sums)."""
+    lengths = [1, 17, 300, 1500, 4000]
+    errors = []
+    for seed in range(4):
+        q, kv, k, v = batch(lengths, 8, 2, d, t.float8_e4m3fn, t.float32, seed=seed)
+        q *= sharp
+        want = reference(q, k, v, lengths)
+        moved = []
+        for x in (kv.k, kv.v):
+            raw = t.empty(x.numel() + 16, dtype=t.uint8, device="cuda")[4:4 + x.numel()]
+            raw.copy_(x.view(t.uint8).flatten())
+            moved.append(raw.view(x.dtype).view(x.shape))
+        other = PagedKVRead(*moved, kv.k_scales, kv.v_scales, kv.block_table, t.arange(len(lengths), device="cuda"),
+                            t.tensor(lengths, dtype=t.int32, device="cuda"), 16)
+        errors.append([float((decode_attention_wrapper(q, x).double() - want).norm() / want.norm()) for x in (kv, other)])
+    ours, valu = (sum(x) for x in zip(*errors))
+    print(f"D {d}, q x {sharp}: {ours / 4:.2e}, vector ALU {valu / 4:.2e}")
+    assert ours <= 1.1 * valu
+
+
 def test_narrow_heads_split_over_the_grid():
     """Enough tokens for every workgroup (and replicas at two KV heads), pages of 32."""
     for hq, hkv in ((32, 8), (8, 2)):
