@@ -104,6 +104,11 @@ class RoPE(nn.Module):
         _native.check(rc, "kvfp8_rope_inplace")
         return x
 
+    @staticmethod
+    def replaced(rope: nn.Module) -> bool:
+        """Whether `rope.apply_` is not this class's: then only it may rotate."""
+        return type(rope) is not RoPE or "apply_" in rope.__dict__
+
     def project(self, x: t.Tensor, weight: t.Tensor, positions: t.Tensor, heads: int) -> t.Tensor:
         """`apply_` of x weight^T, one launch (rows and weights that `_takes_skinny` names)."""
         from aiproj_amd import _native
@@ -206,12 +211,12 @@ class Attention(nn.Module):
         ctx = meta.cache_context
         proj = self.qkv_proj
         # A decode step's rotation is done by the projection's kernel (`kvfp8_skinny_linear_rope`).
-        if (meta.mode != "prefill" and isinstance(proj, RowLinear) and proj.unobserved() and type(self.rope) is RoPE
+        if (meta.mode != "prefill" and isinstance(proj, RowLinear) and proj.unobserved() and not RoPE.replaced(self.rope)
                 and proj.weight.shape[0] == self.q_dim + 2 * self.kv_dim and _takes_skinny(h, proj.weight)):
             qkv = self.rope.project(h, proj.weight, meta.token_positions, cfg.num_q_heads + cfg.num_kv_heads)
             return self._attend(qkv, meta, cache)
         qkv = proj(h)
-        if meta.mode == "prefill":
+        if meta.mode == "prefill" and not RoPE.replaced(self.rope):
             # Prompt attention takes packed q, k and v: rotated and split in one pass.
             split = self.rope.split(qkv, meta.token_positions, cfg.num_q_heads, cfg.num_kv_heads)
             if split is not None:
