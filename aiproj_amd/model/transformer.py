@@ -125,6 +125,8 @@ class RoPE(nn.Module):
         one launch of `rope_vec_kernel`; None for rows it does not take."""
         from aiproj_amd import _native
 
+        if qkv.ndim != 2 or qkv.shape[1] != (num_q_heads + 2 * num_kv_heads) * self.head_dim:
+            return None
         device = _native.require_gpu(qkv, positions, what="rope")
         if qkv.stride(-1) != 1 or not self.cos_table.is_contiguous():
             raise ValueError("rope: rows need unit element stride")

@@ -6,6 +6,7 @@ import types
 import pytest
 import torch as t
 
+from aiproj_amd import _native
 from aiproj_amd.model import transformer
 from aiproj_amd.model.transformer import Attention, ModelConfig, RoPE, StepMeta
 
@@ -74,3 +75,16 @@ def test_a_replaced_rotation_is_used(mode, kind, monkeypatch):
     want = h @ attn.qkv_proj.weight.T
     t.testing.assert_close(q, 2 * want[:, :32].view(5, 4, 8))
     t.testing.assert_close(k, 2 * want[:, 32:48].view(5, 2, 8))
+
+
+@t.no_grad()
+@pytest.mark.parametrize("shape", [(5, 48), (5, 63), (5, 65), (5, 96), (1, 5, 64)])
+def test_rows_of_another_width_do_not_reach_the_split(shape, monkeypatch):
+    """A projection replaced by one of another width or rank: the kernel would read past its rows.
+    It is not called; the views of the separate route judge the rows, as before."""
+    def called():
+        raise AssertionError("the kernel was called")
+
+    monkeypatch.setattr(_native, "require_gpu", lambda *x, what: x[0].device)
+    monkeypatch.setattr(_native, "lib", called)
+    assert RoPE(8, 16, 10000.0).split(t.empty(shape), t.arange(5), 4, 2) is None
