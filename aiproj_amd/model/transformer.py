@@ -173,27 +173,29 @@ def _skinny(entry: str, x: t.Tensor, weight: t.Tensor, columns: int, *more) -> t
     return out
 
 
-def row_linear(x: t.Tensor, weight: t.Tensor) -> t.Tensor:
+def row_linear(x: t.Tensor, weight: t.Tensor, bias: t.Tensor | None = None) -> t.Tensor:
     """x weight^T: the HIP kernel `skinny_linear_kernel` (C ABI `kvfp8_skinny_linear`) for what
-    `_takes_skinny` names, torch's GEMM otherwise."""
+    `_takes_skinny` names, torch's GEMM otherwise and with a bias."""
+    if bias is not None:
+        return F.linear(x, weight, bias)
     if not _takes_skinny(x, weight):
         return F.linear(x, weight)
     return _skinny("kvfp8_skinny_linear", x, weight, weight.shape[0])
 
 
 class RowLinear(nn.Linear):
-    """nn.Linear without bias whose forward is `row_linear`."""
+    """nn.Linear, made without a bias, whose forward is `row_linear`."""
 
     def __init__(self, in_features: int, out_features: int):
         super().__init__(in_features, out_features, bias=False)
 
     def forward(self, x: t.Tensor) -> t.Tensor:
-        return row_linear(x, self.weight)
+        return row_linear(x, self.weight, self.bias)
 
     def unobserved(self) -> bool:
-        """Whether calling the layer does nothing but its own forward: no hook sees its output."""
+        """Whether calling the layer is x weight^T and nothing else: no bias, no hook sees its output."""
         hooks = nn.modules.module
-        return not (type(self) is not RowLinear or "forward" in self.__dict__ or self._forward_hooks
+        return not (type(self) is not RowLinear or "forward" in self.__dict__ or self.bias is not None or self._forward_hooks
                     or self._forward_pre_hooks or hooks._global_forward_hooks or hooks._global_forward_pre_hooks)
 
 

@@ -8,7 +8,7 @@ import torch as t
 
 from aiproj_amd import _native
 from aiproj_amd.model import transformer
-from aiproj_amd.model.transformer import Attention, ModelConfig, RoPE, StepMeta
+from aiproj_amd.model.transformer import Attention, ModelConfig, RoPE, RowLinear, StepMeta, SwiGLU
 
 CFG = ModelConfig(d_model=32, num_q_heads=4, num_kv_heads=2, head_dim=8, d_ff=16, max_seq_len=16)
 
@@ -88,3 +88,38 @@ def test_rows_of_another_width_do_not_reach_the_split(shape, monkeypatch):
     monkeypatch.setattr(_native, "require_gpu", lambda *x, what: x[0].device)
     monkeypatch.setattr(_native, "lib", called)
     assert RoPE(8, 16, 10000.0).split(t.empty(shape), t.arange(5), 4, 2) is None
+
+
+@t.no_grad()
+@pytest.mark.parametrize("mode", ["prefill", "decode"])
+def test_an_assigned_bias_is_added(mode, monkeypatch):
+    """RowLinear is an nn.Linear: a bias that a program gives it counts, also where a decode step's
+    projection would be done by the rotating or the gated kernel."""
+    def kernel(*args):
+        raise AssertionError("the kernel adds no bias")
+
+    monkeypatch.setattr(transformer, "_takes_skinny", lambda x, w: True)
+    monkeypatch.setattr(transformer, "_skinny", kernel)
+    x = t.randn(5, CFG.d_model)
+    layer = RowLinear(CFG.d_model, 24)
+    layer.bias = t.nn.Parameter(t.randn(24))
+    assert t.equal(layer(x), t.nn.functional.linear(x, layer.weight, layer.bias))
+
+    attn = Attention(CFG)
+    attn.rope = Doubling(CFG.head_dim, CFG.max_seq_len, 10000.0)
+    for proj in (attn.qkv_proj, attn.o_proj):
+        proj.bias = t.nn.Parameter(t.randn(proj.out_features))
+    q, _ = attend(attn, mode, monkeypatch, x)
+    t.testing.assert_close(q.flatten(1), 2 * (x @ attn.qkv_proj.weight.T + attn.qkv_proj.bias)[:, :32])
+
+    ffn = SwiGLU(CFG)
+    for proj in (ffn.gate_up, ffn.down):
+        proj.bias = t.nn.Parameter(t.randn(proj.out_features))
+    monkeypatch.setattr(transformer, "silu_mul", lambda gu, n: t.nn.functional.silu(gu[:, :n]) * gu[:, n:])
+    gate, up = (x @ ffn.gate_up.weight.T + ffn.gate_up.bias).chunk(2, -1)
+    t.testing.assert_close(ffn(x), (t.nn.functional.silu(gate) * up) @ ffn.down.weight.T + ffn.down.bias)
+    attn.rope = RoPE(CFG.head_dim, CFG.max_seq_len, 10000.0)
+    monkeypatch.setattr(RoPE, "split", lambda self, qkv, *rest: None)
+    monkeypatch.setattr(RoPE, "apply_", Doubling.apply_)
+    q, _ = attend(attn, mode, monkeypatch, x)
+    t.testing.assert_close(q.flatten(1), 2 * (x @ attn.qkv_proj.weight.T + attn.qkv_proj.bias)[:, :32])
