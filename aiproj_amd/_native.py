@@ -15,6 +15,8 @@ import threading
 from pathlib import Path
 
 import torch
+from torch.overrides import _get_current_function_mode_stack
+from torch.utils._device import DeviceContext
 
 LIBRARY_PATH = Path(__file__).resolve().parent / "libkvfp8.so"
 
@@ -178,9 +180,13 @@ def stream_handle(device: torch.device) -> int:
 
 def is_plain(*tensors: torch.Tensor) -> bool:
     """Tensors whose addresses are their data: no vmap or other transform, mode or trace looks
-    at the operation, which a kernel called with addresses would hide from it."""
+    at the operation, which a kernel called with addresses would hide from it. (A default
+    device is a mode too, which only says where new tensors go.)"""
     if (torch.compiler.is_compiling() or torch.jit.is_tracing() or torch._C._len_torch_dispatch_stack()
-            or torch._C._len_torch_function_stack() or torch.autograd.forward_ad._current_level >= 0):
+            or torch.autograd.forward_ad._current_level >= 0):
+        return False
+    if torch._C._len_torch_function_stack() and any(type(mode) is not DeviceContext
+                                                    for mode in _get_current_function_mode_stack()):
         return False
     wrapped = torch._C._functorch.is_functorch_wrapped_tensor
     return all(type(x) in (torch.Tensor, torch.nn.Parameter) and torch._C._has_storage(x) and not wrapped(x)
