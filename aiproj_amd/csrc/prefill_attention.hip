@@ -1156,18 +1156,17 @@ extern "C" int kvfp8_prefill_attention(const void* q, const void* k, const void*
             default: return (int)launch_generic_prefill<KVFP8_BF16>(a, blocks, s);
         }
     }
-    // 16-bit inputs with D 64, 80, 96, 112 or 128: the wide-tile kernel, whose item and token
-    // indices are int32 (larger inputs take the general kernel below).
+    // 16-bit inputs with D 64, 80, 96, 112 or 128 and scale > 0: the wide-tile kernel, whose item
+    // and token indices are int32 (other inputs take the general kernel below).
     const int fa_rows = kFaRows * kFaWaves / a.heads_per_block;
     const int64_t fa_units = (int64_t)batch * num_kv_heads * a.blocks_per_kv;
     const int64_t fa_upx = (fa_units + kXcds - 1) / kXcds;
     const bool fa_fits = total_tokens < ((int64_t)1 << 31) &&
                          fa_upx * kXcds * (((int64_t)max_seq_len + fa_rows - 1) / fa_rows) < ((int64_t)1 << 31);
-    // Its running maximum of unscaled scores needs scale > 0; 80, 96 and 112 go to the
-    // general kernel otherwise.
-    const bool fa_size = head_dim == 64 || head_dim == 128 ||
-                         (scale > 0.0f && (head_dim == 80 || head_dim == 96 || head_dim == 112));
-    if ((dtype == KVFP8_BF16 || dtype == KVFP8_F16) && fa_size && fa_fits) {
+    // It masks and compares unscaled scores, which needs scale > 0: with a negative one masked
+    // keys would get infinite weight, with 0 NaN. The general kernel scales first.
+    const bool fa_size = head_dim == 64 || head_dim == 80 || head_dim == 96 || head_dim == 112 || head_dim == 128;
+    if ((dtype == KVFP8_BF16 || dtype == KVFP8_F16) && fa_size && fa_fits && scale > 0.0f) {
         a.rows = fa_rows;
         a.qblocks = (max_seq_len + a.rows - 1) / a.rows;
         // One persistent workgroup per CU (its LDS holds one), per_xcd of them on

@@ -35,6 +35,24 @@ def test_wide_kernel_head_sizes(dtype, head_dim, sign):
 
 
 @t.inference_mode()
+@pytest.mark.parametrize("dtype", [t.float16, t.bfloat16])
+@pytest.mark.parametrize("head_dim", [64, 80, 96, 112, 128])
+@pytest.mark.parametrize("scale", [-0.1, 0.0])
+def test_any_scale(dtype, head_dim, scale):
+    """The wide kernel needs a positive scale; others are answered all the same."""
+    lengths = [1, 63, 65, 130]
+    gen = t.Generator(device="cuda").manual_seed(head_dim)
+    q, k, v = (t.randn(sum(lengths), h, head_dim, device="cuda", generator=gen).to(dtype) for h in (8, 2, 2))
+    cu = t.tensor([0] + list(np.cumsum(lengths)), dtype=t.int32, device="cuda")
+    out, lse = flash_attention_forward(q, k, v, cu, max(lengths), scale)
+    want, want_lse = oracle.causal_varlen_attention(*(x.double().cpu().numpy() for x in (q, k, v)), cu.cpu().numpy(),
+                                                    max(lengths), scale)
+    tol = TOLERANCE[dtype]
+    t.testing.assert_close(out.double().cpu(), t.from_numpy(want), rtol=tol, atol=tol)
+    t.testing.assert_close(lse.double().cpu(), t.from_numpy(want_lse), rtol=1e-3, atol=1e-3)
+
+
+@t.inference_mode()
 @pytest.mark.parametrize("dtype,half_ulp", [(t.float16, 2.0 ** -11), (t.bfloat16, 2.0 ** -8)])
 @pytest.mark.parametrize("head_dim", [80, 96, 112])
 def test_largest_probability_is_exact(dtype, half_ulp, head_dim):
