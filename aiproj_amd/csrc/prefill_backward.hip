@@ -72,7 +72,7 @@ struct BwdArgs {
     int32_t cu64;
     int32_t batch, hq, hkv, d;     // d: the caller's head size (<= the kernel's)
     int32_t heads_per_block;       // dQ: q heads per workgroup (4, 2 or 1, dividing G)
-    int32_t key_blocks, q_blocks;  // own blocks of a longest sequence
+    int32_t q_blocks;              // dQ: own blocks of a longest sequence
     int32_t max_len;
     int64_t total_tokens;
     int64_t key_items;             // items of the dK and dV pass
@@ -638,11 +638,12 @@ split_planes_kernel(PlaneArgs a) {
     }
 }
 
-// Layout of the workspace: the two statistics, the sums of split dK and dV, then the
-// planes of q, dO, k, v where the inputs are not read in place.
+// The launches, and the layout of the workspace: the two statistics, the sums of split dK and
+// dV, then the planes of q, dO, k, v where the inputs are not read in place.
 struct BwdPlan {
-    int planes, dp, splits;
+    int planes, dp, splits, waves, heads_per_block;
     bool in_place;
+    int64_t key_items, items, stat_blocks, reduce_blocks;
     int64_t stat, part, q_plane, kv_plane, bytes;
 };
 
@@ -664,19 +665,40 @@ int dkv_splits(int64_t tokens, int32_t batch, int64_t longest, int32_t hq, int32
     return G;
 }
 
-bool plan_backward(int dtype, int64_t tokens, int32_t hq, int32_t hkv, int32_t d, int32_t batch, int32_t max_len,
-                   bool aligned, BwdPlan* p) {
-    if (d < 1 || d > 128) return false;
+int check_backward(int dtype, int64_t tokens, int32_t hq, int32_t hkv, int32_t batch, int32_t max_len) {
+    if (dtype != KVFP8_F32 && dtype != KVFP8_F16 && dtype != KVFP8_BF16) return KVFP8_EDTYPE;
+    return tokens < 0 || batch < 0 || max_len < 0 || hq <= 0 || hkv <= 0 || hq % hkv != 0 ? KVFP8_ESHAPE : KVFP8_OK;
+}
+
+// KVFP8_ELIMIT where a launch would take 2^32 threads or more, which the runtime refuses.
+int plan_backward(int dtype, int64_t tokens, int32_t hq, int32_t hkv, int32_t d, int32_t batch, int32_t max_len,
+                  bool aligned, BwdPlan* p) {
+    if (d < 1 || d > 128) return KVFP8_ESHAPE;
+    if (tokens >= ((int64_t)1 << 31)) return KVFP8_ELIMIT;
+    const int64_t longest = max_len < tokens ? max_len : tokens;
+    const int G = hq / hkv;
     p->planes = dtype == KVFP8_BF16 ? 1 : (dtype == KVFP8_F16 ? 2 : 3);
     p->dp = d <= 64 ? 64 : (d <= 96 ? 96 : 128);
-    p->splits = dkv_splits(tokens, batch, max_len < tokens ? max_len : tokens, hq, hkv);
+    p->waves = p->planes != 2 ? 4 : 8;
+    p->heads_per_block = G % 4 == 0 ? 4 : (G % 2 == 0 ? 2 : 1);
+    p->splits = dkv_splits(tokens, batch, longest, hq, hkv);
+    const int64_t key_rows = 64;                   // four waves' keys
+    const int64_t q_rows = 16 * p->waves / p->heads_per_block;
+    p->key_items = (longest + key_rows - 1) / key_rows * batch * hkv * p->splits;
+    p->items = p->key_items + (longest + q_rows - 1) / q_rows * batch * hkv * (G / p->heads_per_block);
+    p->stat_blocks = (tokens * hq + 15) / 16;
+    p->reduce_blocks = (tokens * hkv * d + 1023) / 1024;
+    const int64_t threads = (int64_t)1 << 32;
+    if (p->items >= threads / (64 * p->waves) || p->stat_blocks >= threads / 256 ||
+        (p->splits > 1 && p->reduce_blocks >= threads / 256))
+        return KVFP8_ELIMIT;
     p->in_place = dtype == KVFP8_BF16 && d == p->dp && aligned;
     p->stat = (tokens * hq * 4 + 255) / 256 * 256;
     p->part = p->splits > 1 ? (2 * p->splits * tokens * hkv * d * 4 + 255) / 256 * 256 : 0;
     p->q_plane = tokens * hq * p->dp * 2;
     p->kv_plane = tokens * hkv * p->dp * 2;
     p->bytes = 2 * p->stat + p->part + (p->in_place ? 0 : 2 * p->planes * (p->q_plane + p->kv_plane));
-    return true;
+    return KVFP8_OK;
 }
 
 template <int D>
@@ -697,14 +719,11 @@ using namespace kvfp8;
 extern "C" int64_t kvfp8_prefill_backward_workspace_bytes(int dtype, int64_t total_tokens, int32_t num_q_heads,
                                                           int32_t num_kv_heads, int32_t head_dim, int32_t batch,
                                                           int32_t max_seq_len, int aligned) {
-    if (dtype != KVFP8_F32 && dtype != KVFP8_F16 && dtype != KVFP8_BF16) return KVFP8_EDTYPE;
-    if (total_tokens < 0 || batch < 0 || max_seq_len < 0 || num_q_heads <= 0 || num_kv_heads <= 0 ||
-        num_q_heads % num_kv_heads != 0)
-        return KVFP8_ESHAPE;
+    int rc = check_backward(dtype, total_tokens, num_q_heads, num_kv_heads, batch, max_seq_len);
+    if (rc != KVFP8_OK) return rc;
     BwdPlan p;
-    if (!plan_backward(dtype, total_tokens, num_q_heads, num_kv_heads, head_dim, batch, max_seq_len, aligned != 0, &p))
-        return KVFP8_ESHAPE;
-    return p.bytes;
+    rc = plan_backward(dtype, total_tokens, num_q_heads, num_kv_heads, head_dim, batch, max_seq_len, aligned != 0, &p);
+    return rc == KVFP8_OK ? p.bytes : rc;
 }
 
 extern "C" int kvfp8_prefill_attention_backward(
@@ -712,11 +731,9 @@ extern "C" int kvfp8_prefill_attention_backward(
     int64_t total_tokens, int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim, const void* cu_seqlens,
     int cu_dtype, int32_t batch, int32_t max_seq_len, float scale, void* dq, void* dk, void* dv, void* workspace,
     int64_t workspace_bytes, void* stream) {
-    if (dtype != KVFP8_F32 && dtype != KVFP8_F16 && dtype != KVFP8_BF16) return KVFP8_EDTYPE;
+    int rc = check_backward(dtype, total_tokens, num_q_heads, num_kv_heads, batch, max_seq_len);
+    if (rc != KVFP8_OK) return rc;
     if (cu_dtype != KVFP8_I32 && cu_dtype != KVFP8_I64) return KVFP8_EDTYPE;
-    if (total_tokens < 0 || batch < 0 || max_seq_len < 0 || num_q_heads <= 0 || num_kv_heads <= 0 ||
-        num_q_heads % num_kv_heads != 0)
-        return KVFP8_ESHAPE;
     if (total_tokens == 0) return KVFP8_OK;
     if (!q || !k || !v || !out || !lse || !grad_out || !dq || !dk || !dv || !workspace || (batch > 0 && !cu_seqlens))
         return KVFP8_ENULL;
@@ -725,26 +742,17 @@ extern "C" int kvfp8_prefill_attention_backward(
     if (((inputs | (uintptr_t)out) & element) != 0) return KVFP8_ESTRIDE;
     if ((((uintptr_t)dq | (uintptr_t)dk | (uintptr_t)dv | (uintptr_t)workspace) & 15) != 0) return KVFP8_ESTRIDE;
     BwdPlan plan;
-    if (!plan_backward(dtype, total_tokens, num_q_heads, num_kv_heads, head_dim, batch, max_seq_len, (inputs & 15) == 0,
-                       &plan))
-        return KVFP8_ESHAPE;
+    rc = plan_backward(dtype, total_tokens, num_q_heads, num_kv_heads, head_dim, batch, max_seq_len, (inputs & 15) == 0,
+                       &plan);
+    if (rc != KVFP8_OK) return rc;
     if (workspace_bytes < plan.bytes) return KVFP8_EWORKSPACE;
-    if (total_tokens >= ((int64_t)1 << 31)) return KVFP8_ELIMIT;
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     uint8_t* ws = reinterpret_cast<uint8_t*>(workspace);
 
     BwdArgs a;
-    const int G = num_q_heads / num_kv_heads;
-    a.heads_per_block = G % 4 == 0 ? 4 : (G % 2 == 0 ? 2 : 1);
-    const int waves = plan.planes != 2 ? 4 : 8;
-    const int64_t longest = max_seq_len < total_tokens ? max_seq_len : total_tokens;
-    const int key_rows = 64;                       // four waves' keys
-    const int64_t key_blocks = (longest + key_rows - 1) / key_rows;
-    const int64_t q_rows = 16 * waves / a.heads_per_block, q_blocks = (longest + q_rows - 1) / q_rows;
+    a.heads_per_block = plan.heads_per_block;
     a.splits = plan.splits;
-    a.key_items = key_blocks * batch * num_kv_heads * a.splits;
-    const int64_t items = a.key_items + q_blocks * batch * num_kv_heads * (G / a.heads_per_block);
-    if (items >= ((int64_t)1 << 31)) return KVFP8_ELIMIT;
+    a.key_items = plan.key_items;
 
     StatArgs st;
     st.out = out;
@@ -765,9 +773,7 @@ extern "C" int kvfp8_prefill_attention_backward(
     st.total_tokens = total_tokens;
     st.splits = plan.splits;
     st.part = a.part = reinterpret_cast<float*>(ws + 2 * plan.stat);
-    const int64_t stat_blocks = (total_tokens * num_q_heads + 15) / 16;
-    if (stat_blocks >= ((int64_t)1 << 31)) return KVFP8_ELIMIT;
-    const dim3 stat_grid((unsigned)stat_blocks), block(256);
+    const dim3 stat_grid((unsigned)plan.stat_blocks), block(256);
     const int32_t vec = (head_dim * (dtype == KVFP8_F32 ? 4 : 2)) % 16 == 0 && (((uintptr_t)out | (uintptr_t)grad_out) & 15) == 0;
     switch (dtype) {
         case KVFP8_F32: hipLaunchKernelGGL((bwd_stats_kernel<KVFP8_F32>), stat_grid, block, 0, s, st, vec); break;
@@ -775,7 +781,7 @@ extern "C" int kvfp8_prefill_attention_backward(
         default: hipLaunchKernelGGL((bwd_stats_kernel<KVFP8_BF16>), stat_grid, block, 0, s, st, vec); break;
     }
     hipError_t err = hipGetLastError();
-    if (err != hipSuccess || items == 0) return (int)err;
+    if (err != hipSuccess || plan.items == 0) return (int)err;
 
     a.q = reinterpret_cast<const uint8_t*>(q);
     a.k = reinterpret_cast<const uint8_t*>(k);
@@ -823,20 +829,21 @@ extern "C" int kvfp8_prefill_attention_backward(
     a.hq = num_q_heads;
     a.hkv = num_kv_heads;
     a.d = head_dim;
-    a.key_blocks = (int32_t)key_blocks;
-    a.q_blocks = (int32_t)q_blocks;
+    const int64_t longest = max_seq_len < total_tokens ? max_seq_len : total_tokens;
+    const int64_t q_rows = 16 * plan.waves / plan.heads_per_block;
+    a.q_blocks = (int32_t)((longest + q_rows - 1) / q_rows);
     a.max_len = max_seq_len;
     a.total_tokens = total_tokens;
     a.scale = scale;
     a.scale_log2 = scale * 1.44269504088896340736f;
     switch (plan.dp) {
-        case 64: err = launch_backward<64>(a, plan.planes, items, s); break;
-        case 96: err = launch_backward<96>(a, plan.planes, items, s); break;
-        default: err = launch_backward<128>(a, plan.planes, items, s); break;
+        case 64: err = launch_backward<64>(a, plan.planes, plan.items, s); break;
+        case 96: err = launch_backward<96>(a, plan.planes, plan.items, s); break;
+        default: err = launch_backward<128>(a, plan.planes, plan.items, s); break;
     }
     if (err != hipSuccess || plan.splits == 1) return (int)err;
     const int64_t count = total_tokens * num_kv_heads * head_dim;
-    const dim3 grid((unsigned)((count + 1023) / 1024), 2);
+    const dim3 grid((unsigned)plan.reduce_blocks, 2);
     switch (dtype) {
         case KVFP8_F32: hipLaunchKernelGGL((bwd_reduce_kernel<KVFP8_F32>), grid, block, 0, s, a.part, count, plan.splits, scale, dk, dv); break;
         case KVFP8_F16: hipLaunchKernelGGL((bwd_reduce_kernel<KVFP8_F16>), grid, block, 0, s, a.part, count, plan.splits, scale, dk, dv); break;

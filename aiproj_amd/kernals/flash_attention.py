@@ -86,6 +86,9 @@ def _native_backward(q, k, v, output, lse, cum_seq, grad_output, batch_max_seq_l
     batch, longest = cum_seq.shape[0] - 1, int(batch_max_seq_len)
     aligned = all(x.data_ptr() % 16 == 0 for x in (q, k, v, grad_output))
     size = _native.lib().kvfp8_prefill_backward_workspace_bytes(code, total, hq, hkv, d, batch, longest, aligned)
+    if size == _native.ELIMIT:
+        return None
+    _native.check(min(size, 0), "kvfp8_prefill_backward_workspace_bytes")
     dq, dk, dv = t.empty_like(q), t.empty_like(k), t.empty_like(v)
     workspace = t.empty(size, dtype=t.uint8, device=q.device)
     rc = _native.lib().kvfp8_prefill_attention_backward(
@@ -93,8 +96,6 @@ def _native_backward(q, k, v, output, lse, cum_seq, grad_output, batch_max_seq_l
         total, hq, hkv, d, cum_seq.data_ptr(), _native.dtype_code(cum_seq.dtype), batch,
         longest, float(scale), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), workspace.data_ptr(), size,
         _native.stream_handle(q.device))
-    if rc == _native.ELIMIT:      # returned before anything is launched
-        return None
     _native.check(rc, "kvfp8_prefill_attention_backward")
     return dq, dk, dv
 

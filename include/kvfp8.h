@@ -257,6 +257,7 @@ int kvfp8_prefill_attention(const void* q_dev, const void* k_dev, const void* v_
  * max_seq_len of theirs, get zeros. head_dim 1..128. Results do not depend on timing.
  *   workspace: kvfp8_prefill_backward_workspace_bytes(...) bytes, 16-byte aligned, any
  *   contents; `aligned`: q, k, v and grad_out are 16-byte aligned (fewer bytes then). dq, dk and dv are 16-byte aligned.
+ * Both return KVFP8_ELIMIT where a launch would take 2^32 threads or more.
  * Replaces the backward of reference src/torch_llm/kernals/flash_attention.py:213 onwards.
  */
 int64_t kvfp8_prefill_backward_workspace_bytes(int dtype, int64_t total_tokens, int32_t num_q_heads,

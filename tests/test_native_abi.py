@@ -292,3 +292,22 @@ def test_fast_bindings_match_ctypes_on_host_checks(lib):
         assert fast.kvfp8_store_append(*args) == lib.kvfp8_store_append(*args) < 0, args
     with pytest.raises(TypeError):
         fast.kvfp8_quantize_append(*append, 0)
+
+
+@pytest.mark.parametrize("dtype,total,hq,batch,longest", [
+    (_native.BF16, 2 ** 24, 16, 1, 64),                # row statistics: 2^24 workgroups of 256 threads
+    (_native.BF16, 2 ** 20, 4, 2 ** 11, 2 ** 20),      # items of a loose longest length: 2^25 and more
+    (_native.F16, 2 ** 20, 1, 2 ** 8, 2 ** 20),        # 2^22 of dK and dV and 2^21 of dQ, 512 threads each
+    (_native.F16, 2 ** 20, 1, 2 ** 9, 2 ** 20),
+])
+def test_attention_backward_refuses_grids_beyond_the_runtime(lib, dtype, total, hq, batch, longest):
+    """2^32 threads or more: KVFP8_ELIMIT before any launch (callers then take another way), also from
+    the workspace size. The pointers are never read."""
+    size = lib.kvfp8_prefill_backward_workspace_bytes(dtype, total, hq, 1, 64, batch, longest, 1)
+    if batch == 2 ** 8:
+        assert size > 0                                # just below
+        return
+    assert size == _native.ELIMIT
+    p = 4096
+    assert lib.kvfp8_prefill_attention_backward(p, p, p, p, p, p, dtype, total, hq, 1, 64, p, _native.I32, batch,
+                                                longest, 1.0, p, p, p, p, 2 ** 62, None) == _native.ELIMIT
