@@ -17,8 +17,8 @@ Same interface as the reference:
 The backward (`flash_attention_backward`, reference `:213-...`) is one call of the HIP
 kernels behind `kvfp8_prefill_attention_backward` for head sizes up to 128: products of
 float32 accuracy on the matrix cores, no host synchronization. Other head sizes, mixed
-dtypes, strided inputs and CPU tensors take PyTorch float32 operations, sequence by
-sequence (that path reads the sequence bounds on the host).
+dtypes, strided inputs, CPU tensors and calls that are to be differentiated take PyTorch
+float32 operations, sequence by sequence (that path reads the sequence bounds on the host).
 
 Head sizes 1 to 512 (`ValueError` otherwise), like the reference, which pads any size
 to a power of two (`:72`): multiples of 8 up to 128 run on the matrix-core kernels, every
@@ -69,7 +69,7 @@ _MAX_BACKWARD_HEAD = 128
 def _native_backward(q, k, v, output, lse, cum_seq, grad_output, batch_max_seq_len, scale):
     """dq, dk, dv from the HIP kernels, or None for what they do not take."""
     rows = (q, k, v, output, grad_output)
-    if not _native.is_plain(*rows, lse, cum_seq):
+    if not _native.is_plain(*rows, lse, cum_seq) or (t.is_grad_enabled() and any(x.requires_grad for x in (*rows, lse))):
         return None
     if (q.device.type != "cuda" or q.dtype not in _DTYPES or q.ndim != 3 or q.shape[2] > _MAX_BACKWARD_HEAD
             or q.numel() == 0 or lse.dtype != t.float32 or cum_seq.dtype not in (t.int32, t.int64) or cum_seq.ndim != 1

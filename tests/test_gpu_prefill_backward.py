@@ -7,6 +7,7 @@ import math
 import pytest
 import torch as t
 
+from aiproj_amd import _native
 from aiproj_amd.kernals import flash_attention as fa
 
 pytestmark = pytest.mark.gpu
@@ -133,3 +134,32 @@ def test_float32_is_no_less_exact_than_torch(d, positive):
     torch_got = fa.flash_attention_backward(q, k, v, out, lse, cu, strided, max(lengths), scale)
     for g, x, w in zip(got, torch_got, reference(q, k, v, bounds, max(lengths), grad)):
         assert float((g.double() - w).norm()) <= 1.1 * float((x.double() - w).norm())
+
+
+def test_a_backward_that_is_differentiated_is_recorded():
+    """flash_attention_backward called on tensors that require gradients: PyTorch operations, whose
+    graph the kernels would cut off. dq is linear in grad_output."""
+    bounds, (q, k, v, grad) = inputs([33, 70], 4, 2, 64, t.float32)
+    cu = t.tensor(bounds, dtype=t.int32, device="cuda")
+    out, lse = fa.flash_attention_forward(q, k, v, cu, 70, 0.125)
+    want = fa.flash_attention_backward(q, k, v, out, lse, cu, grad, 70, 0.125)
+    got = fa.flash_attention_backward(q, k, v, out, lse, cu, grad.requires_grad_(True), 70, 0.125)
+    check([g.detach() for g in got], [w.double() for w in want], t.float32)
+    direction, = t.autograd.grad(got[0], grad, want[0])
+    t.testing.assert_close((direction * grad).sum(), (want[0] * want[0]).sum(), rtol=1e-4, atol=0)
+    with t.no_grad():
+        again = fa.flash_attention_backward(q, k, v, out, lse, cu, grad, 70, 0.125)
+    assert all(t.equal(a, w) for a, w in zip(again, want))
+
+
+def test_a_refused_size_takes_the_pytorch_operations(monkeypatch):
+    bounds, (q, k, v, grad) = inputs([33, 70], 4, 2, 64, t.float16)
+    cu = t.tensor(bounds, dtype=t.int32, device="cuda")
+    out, lse = fa.flash_attention_forward(q, k, v, cu, 70, 0.125)
+
+    class Refusing:
+        def kvfp8_prefill_backward_workspace_bytes(self, *args):
+            return _native.ELIMIT
+
+    monkeypatch.setattr(_native, "lib", Refusing)
+    check(fa.flash_attention_backward(q, k, v, out, lse, cu, grad, 70, 0.125), reference(q, k, v, bounds, 70, grad), t.float16)
