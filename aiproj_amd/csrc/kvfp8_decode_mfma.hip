@@ -1171,19 +1171,6 @@ int ilog2(int64_t x) {
 // Waves that serve distinct KV heads: one per head, up to kMaxWaves.
 int waves_for(int32_t num_kv_heads) { return num_kv_heads < kMaxWaves ? num_kv_heads : kMaxWaves; }
 
-// Compute units of the current device (cached per device id).
-int device_cus() {
-    static int cus[64] = {0};
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-    if (cus[dev] == 0) {
-        int n = 0;
-        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
-        cus[dev] = n;
-    }
-    return cus[dev];
-}
-
 // Fewer KV heads than kMaxWaves, dividing it: the plain decode runs kMaxWaves waves per
 // workgroup, R = kMaxWaves / heads replicas of each head (kRep), when
 //   - the replicas' merge buffer fits in LDS beside the batch-sized tables, and

@@ -966,19 +966,6 @@ prefill_fa_kernel(PrefillArgs a, int32_t units, int32_t upx, int32_t per_xcd) {
     }
 }
 
-// Compute units of the current device (cached per device id).
-int fa_device_cus() {
-    static int cus[64] = {};
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 0;
-    if (cus[dev] == 0) {
-        int n = 0;
-        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
-        cus[dev] = n;
-    }
-    return cus[dev];
-}
-
 // ---------------------------------------------------------------------------
 // Vector-ALU kernel for the head sizes the matrix-core kernels do not take (not a
 // multiple of 8, or above 128; up to kGenMaxD), as the reference's Triton kernel
@@ -1174,7 +1161,7 @@ extern "C" int kvfp8_prefill_attention(const void* q, const void* k, const void*
         const int64_t units = fa_units;
         const int64_t upx = fa_upx;
         const int64_t items_per_xcd = upx * (int64_t)a.qblocks;
-        int64_t per_xcd = fa_device_cus() / kXcds;
+        int64_t per_xcd = device_cus() / kXcds;
         per_xcd = per_xcd < 1 ? 1 : per_xcd;
         per_xcd = per_xcd < items_per_xcd ? per_xcd : items_per_xcd;
         const dim3 grid((unsigned)(kXcds * per_xcd));

@@ -649,19 +649,29 @@ struct BwdPlan {
 
 // Workgroups per KV head and key block for dK and dV. One workgroup for all G q heads needs
 // no second pass, but its chain of G * len / 32 steps then bounds the launch unless the
-// batch keeps every CU busy for longer; a split writes float32 sums that a second pass adds
-// in order. The batch's steps per CU (64 keys x 32 rows; dQ adds about 0.6) are estimated at
-// the mean length, and the smallest split is taken whose chain, at 1.75 times a CU's rate,
-// fits under them. Measured with 16q/4kv heads, D 128, bf16 (us at 1, 2 and 4 workgroups): 4
-// sequences of 1024 tokens 248, 151, 135 (takes 4); 8: 279, 241, 262 (takes 2); 16: 503 at
-// 2, 521 at 1 (takes 1); 16 of 64 to 1024 tokens 269, 286, 313 (takes 2: lengths are not
-// known on the host).
-int dkv_splits(int64_t tokens, int32_t batch, int64_t longest, int32_t hq, int32_t hkv) {
+// batch keeps every CU busy for longer; a split writes float32 sums (up to four times q's bytes)
+// that a second pass adds in order. The smallest split is taken whose chain fits under the rest,
+// in steps of a CU (64 keys x 32 rows; dQ adds about 0.6):
+// - the pairs at the mean length, or those of the longest sequence where they are more (lengths
+//   are not known on the host, only their sum and their limit);
+// - the dispatch of `items` workgroups, of which most are empty where lengths are uneven: 1.4 to
+//   4 ns each, about 400 a step.
+// A chain's step takes 1.75 times a CU's where three workgroups share one (bf16), else as long.
+// Measured with 1, 2 and 4 workgroups (us; * taken). 16q/4kv heads, D 128, bf16: 4 sequences of
+// 1024 tokens 257, 154, 138*; 8: 289, 245*, 270; 16: 455*, 504, 554; 16 of 64 to 1024: 292, 277*,
+// 297; 300 of 64 with a limit of 4096 675*, 828, 1060; 60 of 128 and one of 4096 1001, 860*, 931.
+// float16, 4 of 1024 287, 292*, 308; 8 574*, 601, 648; float32, 8 1091*, 1116, 1160. 8q/2kv, D 64,
+// bf16: 16 of 1024 184, 142*, 152; 300 of 64 and one of 1024 194, 153, 181*. Over 123 batches of
+// five head layouts the choice costs 2.1% more than the best one, at most 30%; at the mean length
+// alone and 1.75 for every type it cost 8.8%, at most 85%.
+int dkv_splits(int64_t tokens, int32_t batch, int64_t longest, int32_t hq, int32_t hkv, int planes, int64_t items) {
     const int G = hq / hkv;
-    const double mean = batch > 0 ? (double)tokens / batch : 0.0;
-    const double busy = 1.6 * hq * (double)tokens * mean / 2 / (64 * 32) / 256;
+    double squares = batch > 0 ? (double)tokens * (double)tokens / batch : 0.0;
+    squares = squares > (double)longest * longest ? squares : (double)longest * longest;
+    const double busy = 1.6 * hq * squares / 2 / (64 * 32) / device_cus() + (double)items / 400;
+    const double step = planes == 1 ? 1.75 : 1.0;
     for (int n = 1; n < G; ++n)
-        if (G % n == 0 && (double)(G / n) * (double)longest / 32 * 1.75 <= busy) return n;
+        if (G % n == 0 && (double)(G / n) * (double)longest / 32 * step <= busy) return n;
     return G;
 }
 
@@ -681,11 +691,13 @@ int plan_backward(int dtype, int64_t tokens, int32_t hq, int32_t hkv, int32_t d,
     p->dp = d <= 64 ? 64 : (d <= 96 ? 96 : 128);
     p->waves = p->planes != 2 ? 4 : 8;
     p->heads_per_block = G % 4 == 0 ? 4 : (G % 2 == 0 ? 2 : 1);
-    p->splits = dkv_splits(tokens, batch, longest, hq, hkv);
     const int64_t key_rows = 64;                   // four waves' keys
     const int64_t q_rows = 16 * p->waves / p->heads_per_block;
-    p->key_items = (longest + key_rows - 1) / key_rows * batch * hkv * p->splits;
-    p->items = p->key_items + (longest + q_rows - 1) / q_rows * batch * hkv * (G / p->heads_per_block);
+    const int64_t key_items = (longest + key_rows - 1) / key_rows * batch * hkv;
+    const int64_t q_items = (longest + q_rows - 1) / q_rows * batch * hkv * (G / p->heads_per_block);
+    p->splits = dkv_splits(tokens, batch, longest, hq, hkv, p->planes, key_items + q_items);
+    p->key_items = key_items * p->splits;
+    p->items = p->key_items + q_items;
     p->stat_blocks = (tokens * hq + 15) / 16;
     p->reduce_blocks = (tokens * hkv * d + 1023) / 1024;
     const int64_t threads = (int64_t)1 << 32;

@@ -249,18 +249,6 @@ skinny_linear_kernel(LinArgs a) {
     }
 }
 
-int linear_cus() {
-    static int cus[64] = {};
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 0;
-    if (cus[dev] == 0) {
-        int n = 0;
-        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
-        cus[dev] = n;
-    }
-    return cus[dev];
-}
-
 template <int MT, int STEPS>
 hipError_t launch_linear(const LinArgs& a, bool f16, int grid, hipStream_t s) {
     const dim3 g(grid), b(64 * kLinWaves);
@@ -316,7 +304,7 @@ int skinny_linear(LinArgs a, const void* x, int dtype, int64_t x_stride, int32_t
     int per_wave = 2;
     while (per_wave < kLinSteps && kLinWaves * per_wave < a.steps) per_wave *= 2;
     a.groups = (a.steps + kLinWaves * per_wave - 1) / (kLinWaves * per_wave);
-    const int cus = linear_cus();
+    const int cus = device_cus();
     // Row tiles per workgroup: all of them, or fewer while that puts idle CUs to work.
     int mt = (rows + 15) / 16;
     const int row_tiles = mt;

@@ -311,3 +311,23 @@ def test_attention_backward_refuses_grids_beyond_the_runtime(lib, dtype, total, 
     p = 4096
     assert lib.kvfp8_prefill_attention_backward(p, p, p, p, p, p, dtype, total, hq, 1, 64, p, _native.I32, batch,
                                                 longest, 1.0, p, p, p, p, 2 ** 62, None) == _native.ELIMIT
+
+
+@pytest.mark.parametrize("dtype,hq,hkv,d,batch,total,longest,splits", [
+    (_native.BF16, 16, 4, 128, 1, 1024, 1024, 4),
+    (_native.BF16, 16, 4, 128, 4, 4096, 1024, 4),
+    (_native.BF16, 16, 4, 128, 8, 8192, 1024, 2),
+    (_native.BF16, 16, 4, 128, 16, 16384, 1024, 1),
+    (_native.BF16, 16, 4, 128, 16, 8704, 1024, 2),
+    (_native.F16, 16, 4, 128, 8, 8192, 1024, 1),           # one workgroup per CU: its chain is no slower
+    (_native.BF16, 64, 8, 128, 1000, 64000, 8192, 1),      # short sequences under a far limit
+    (_native.BF16, 16, 4, 128, 300, 300 * 64, 4096, 1),
+    (_native.BF16, 8, 2, 64, 61, 60 * 128 + 4096, 4096, 4),
+])
+def test_attention_backward_splits_where_it_was_measured_to_pay(lib, dtype, hq, hkv, d, batch, total, longest, splits):
+    """The workgroups that share a KV head's q heads, from the partial sums in the workspace (256 CUs:
+    the count where no device is, too)."""
+    size = lib.kvfp8_prefill_backward_workspace_bytes(dtype, total, hq, hkv, d, batch, longest, 1)
+    stats = 2 * (-(-total * hq * 4 // 256) * 256)
+    planes = {_native.BF16: 0, _native.F16: 2}[dtype] * 2 * 2 * total * (hq + hkv) * d
+    assert size - stats - planes == (0 if splits == 1 else 2 * splits * total * hkv * d * 4)
