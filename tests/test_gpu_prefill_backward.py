@@ -67,7 +67,7 @@ def test_backward_matches_float64(dtype, hq, hkv, d):
 
 @pytest.mark.parametrize("count", [1, 8, 24])
 def test_backward_splits_over_q_heads(count):
-    """One long sequence to many: every number of workgroups per KV head, twice the same bits."""
+    """One long sequence to many (4, 4 and 2 workgroups per KV head), twice the same bits."""
     lengths = [520] * count
     bounds, (q, k, v, grad) = inputs(lengths, 8, 2, 64, t.bfloat16, seed=count)
     cu = t.tensor(bounds, dtype=t.int64, device="cuda")
@@ -163,3 +163,25 @@ def test_a_refused_size_takes_the_pytorch_operations(monkeypatch):
 
     monkeypatch.setattr(_native, "lib", Refusing)
     check(fa.flash_attention_backward(q, k, v, out, lse, cu, grad, 70, 0.125), reference(q, k, v, bounds, 70, grad), t.float16)
+
+
+@pytest.mark.parametrize("dtype,count,splits", [
+    (t.bfloat16, 1, 4), (t.bfloat16, 24, 2), (t.bfloat16, 40, 1), (t.float16, 1, 4), (t.float16, 10, 2),
+    (t.float16, 24, 1), (t.float32, 1, 4), (t.float32, 10, 2), (t.float32, 24, 1)])
+def test_every_split_of_four_q_heads(dtype, count, splits):
+    """4, 2 and 1 workgroups per KV head and key block, the last one storing dK and dV itself after a
+    chain over all four q heads. The workspace's partial sums say which split was taken."""
+    hq, hkv, d, longest = 8, 2, 64, 520
+    total = longest * count
+    size = _native.lib().kvfp8_prefill_backward_workspace_bytes(_native.dtype_code(dtype), total, hq, hkv, d, count,
+                                                                longest, 1)
+    planes = {t.bfloat16: 0, t.float16: 2, t.float32: 3}[dtype]
+    rest = 2 * (-(-total * hq * 4 // 256) * 256) + 2 * planes * total * (hq + hkv) * d * 2
+    assert size - rest == (0 if splits == 1 else 2 * splits * total * hkv * d * 4)
+    bounds, (q, k, v, grad) = inputs([longest] * count, hq, hkv, d, dtype, seed=count)
+    cu = t.tensor(bounds, dtype=t.int32, device="cuda")
+    out, lse = fa.flash_attention_forward(q, k, v, cu, longest, 0.125)
+    got = fa._native_backward(q, k, v, out, lse, cu, grad, longest, 0.125)
+    check(got, reference(q, k, v, bounds, longest, grad), dtype)
+    again = fa._native_backward(q, k, v, out, lse, cu, grad, longest, 0.125)
+    assert all(t.equal(a, b) for a, b in zip(got, again))
