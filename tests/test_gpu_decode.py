@@ -209,10 +209,10 @@ def test_decode_edge_cases_and_calling_forms():
 @t.inference_mode()
 @pytest.mark.parametrize("head_dim", [64, 80])
 def test_decode_block_sizes_other_than_16(head_dim):
-    # D 64: page sizes under 16 take the VALU kernel, 32 and up the MFMA kernel; D 80
-    # always the grouped VALU kernel. Pages of 1 and 2 fill its whole per-wave page
-    # list (256 entries for a 256-token chunk); pages of 256 and 512 hold a whole chunk
-    # (one entry), and lengths past 600 cross pages and chunks.
+    # Page sizes under 16 take the grouped VALU kernel, 32 and up the MFMA kernel (D 80 as
+    # narrow rows; the grouped kernel's large pages: test_grouped_kernel_at_head_size_80).
+    # Pages of 1 and 2 fill the grouped kernel's whole per-wave page list (256 entries
+    # for a 256-token chunk), and lengths past 600 cross pages and chunks.
     for block_size in (1, 2, 4, 8, 32, 64, 256, 512):
         lengths = [3, 40, 129, 700]
         cache = PagedKVCache(sum(-(-n // block_size) for n in lengths) + 4, block_size, 2, head_dim, "cuda", FP8)
@@ -269,14 +269,37 @@ def test_unaligned_caches_take_the_valu_kernels(offset, cache_dtype, q_dtype):
 @t.inference_mode()
 @pytest.mark.parametrize("num_q_heads,num_kv_heads", [(32, 1), (12, 2), (6, 6)])
 def test_valu_kernel_head_groups(num_q_heads, num_kv_heads):
-    # D 80 (no MFMA kernel): groups of 32, 6 and 1 q heads per KV head, which the
-    # grouped kernel splits into balanced sets of at most four heads per wave.
+    # D 80: a group of 32 q heads per KV head, which the grouped kernel splits into balanced
+    # sets of at most four heads per wave; groups of 6 and 1 on the MFMA kernel's narrow rows
+    # (the grouped kernel's: test_grouped_kernel_at_head_size_80).
     lengths = [2, 33, 300, 900]
     d = 80
     cache = PagedKVCache(sum(-(-n // 16) for n in lengths) + 4, 16, num_kv_heads, d, "cuda", FP8)
     manager, context, _, _ = fill_decode_batch([cache], lengths, num_kv_heads, d, 16, t.bfloat16, seed=17)
     q = t.randn(len(lengths), num_q_heads, d, device="cuda", dtype=t.float32)
     actual = decode_attention_wrapper(q, cache, context)
+    expected = oracle_decode(q, cache, manager.block_table, context.cache_slots, lengths)
+    t.testing.assert_close(actual.double().cpu(), t.from_numpy(expected), rtol=1e-4, atol=1e-4)
+
+
+@t.inference_mode()
+@pytest.mark.parametrize("num_q_heads,num_kv_heads,block_size,lengths", [
+    (12, 2, 16, [2, 33, 300, 900]),                     # sets of three and three heads per wave
+    (6, 6, 16, [2, 33, 300, 900]),                      # one head per wave
+    (8, 2, 32, [3, 40, 129, 700]),
+    (8, 2, 256, [3, 40, 129, 700, 1100]),               # a page holds a whole chunk
+    (8, 2, 512, [3, 40, 129, 700, 1100]),
+])
+def test_grouped_kernel_at_head_size_80(num_q_heads, num_kv_heads, block_size, lengths):
+    """Caches 4 bytes past a 16-byte boundary, which the MFMA kernel does not take: the grouped kernel's
+    slices of 20 at uneven head groups and at pages of a chunk and more."""
+    d = 80
+    cache = PagedKVCache(sum(-(-n // block_size) for n in lengths) + 4, block_size, num_kv_heads, d, "cuda", FP8)
+    manager, context, _, _ = fill_decode_batch([cache], lengths, num_kv_heads, d, block_size, t.bfloat16, seed=17)
+    q = t.randn(len(lengths), num_q_heads, d, device="cuda", dtype=t.float32)
+    read = PagedKVRead(_shifted(cache.k, 4), _shifted(cache.v, 4), cache.k_scales, cache.v_scales,
+                       manager.block_table, context.cache_slots, context.context_lengths, block_size)
+    actual = decode_attention_wrapper(q, read)
     expected = oracle_decode(q, cache, manager.block_table, context.cache_slots, lengths)
     t.testing.assert_close(actual.double().cpu(), t.from_numpy(expected), rtol=1e-4, atol=1e-4)
 
@@ -595,7 +618,8 @@ def test_replicated_heads(hq, hkv, d, batch, long_len, cache_dtype, block_size):
 def test_maximum_batch(head_dim):
     """8,191 sequences, the most the decode kernels' LDS tile prefix holds (8,192 is
     refused on the host, tests/test_native_abi.py): D 64 on the MFMA kernel (its
-    prefix and sequence metadata take 64 KB of LDS), D 80 on the grouped VALU kernel.
+    prefix and sequence metadata take 64 KB of LDS), D 80 on its narrow rows (and the
+    same bytes 4 off a 16-byte boundary on the grouped VALU kernel).
     Every row against float32 dequantize-then-attend, sampled rows against the oracle."""
     from tests.helpers import torch_paged_decode
 
@@ -612,6 +636,11 @@ def test_maximum_batch(head_dim):
     assert t.isfinite(out).all()
     ref = torch_paged_decode(w.q, cache, w.cache_slots, ctx.context_lengths, w.block_table)
     t.testing.assert_close(out.float(), ref, rtol=NORTH_STAR_RTOL, atol=NORTH_STAR_ATOL)
+    if head_dim == 80:
+        read = PagedKVRead(_shifted(cache.k, 4), _shifted(cache.v, 4), cache.k_scales, cache.v_scales, w.block_table,
+                           ctx.cache_slots, ctx.context_lengths, 16)
+        t.testing.assert_close(decode_attention_wrapper(w.q, read).float(), ref, rtol=NORTH_STAR_RTOL,
+                               atol=NORTH_STAR_ATOL)
     rows = [0, 1, 4095, batch - 1]
     expected = oracle_decode(w.q, cache, w.block_table, w.cache_slots, lengths, rows=rows)
     t.testing.assert_close(out[rows].double().cpu(), t.from_numpy(expected), rtol=NORTH_STAR_RTOL,

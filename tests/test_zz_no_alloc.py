@@ -77,7 +77,8 @@ def test_noalloc_with_replicated_heads():
 @pytest.mark.gpu
 @t.inference_mode()
 def test_noalloc_on_the_generic_kernel():
-    """Head size 80 and an f32 cache take the VALU kernel and its own workspace layout."""
+    """An f32 cache takes the VALU kernel and its own workspace layout; head size 80 the narrow rows of the
+    MFMA kernel."""
     lengths = [1, 300, 17, 1000]
     for dtype, d, hq, hkv in ((t.float8_e4m3fn, 80, 8, 2), (t.float32, 64, 8, 2)):
         spec = workloads.WorkloadSpec("generic", len(lengths), hq, hkv, d, lengths, seed=51)
