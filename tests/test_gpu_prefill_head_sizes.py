@@ -36,10 +36,11 @@ def test_wide_kernel_head_sizes(dtype, head_dim, sign):
 
 @t.inference_mode()
 @pytest.mark.parametrize("dtype", [t.float16, t.bfloat16])
-@pytest.mark.parametrize("head_dim", [64, 80, 96, 112, 128])
-@pytest.mark.parametrize("scale", [-0.1, 0.0])
+@pytest.mark.parametrize("head_dim,scale", [(d, s) for d in (64, 80, 96, 112, 128) for s in (-0.1, 0.0)]
+                         + [(72, 0.1), (88, 0.1), (104, 0.1), (120, -0.1)])
 def test_any_scale(dtype, head_dim, scale):
-    """The wide kernel needs a positive scale; others are answered all the same."""
+    """What the wide kernel leaves to the general one, on its rows of 64 and of 128 dims: scales that are
+    not positive, and the other multiples of 8."""
     lengths = [1, 63, 65, 130]
     gen = t.Generator(device="cuda").manual_seed(head_dim)
     q, k, v = (t.randn(sum(lengths), h, head_dim, device="cuda", generator=gen).to(dtype) for h in (8, 2, 2))
