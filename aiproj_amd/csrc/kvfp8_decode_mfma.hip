@@ -1083,9 +1083,13 @@ __device__ __forceinline__ int32_t group_of(int64_t x, int64_t total, int64_t gr
 //   out = den > 0 ? num / den : 0. Empty sequences get zeros.
 // One wave per (sequence, q head). Piece states are read lane-parallel (m and l
 // one piece per lane, acc as float4 runs with D/4 lanes per piece), so the merge
-// costs a couple of memory latencies whatever the number of pieces.
+// costs a couple of memory latencies for the pieces of an ordinary batch.
 // Narrow rows take the lanes of 128 dims per piece; those past the row only follow.
-template <int C, int QT, bool kNarrow>
+// kShare (narrow rows, fewer pairs than the chip has SIMDs): the four waves of a workgroup
+// share a pair's pieces, of which a lone long sequence has hundreds. One sequence of 20000
+// tokens, D 80, decode and combine, 4q/1kv and 8q/2kv heads: 51 and 47 us with a wave per pair
+// (37 and 38 on the vector ALU) -> 21 us; 1 to 16 sequences of 500: 9 to 14 us both.
+template <int C, int QT, bool kNarrow, bool kShare>
 __global__ void __launch_bounds__(256)
 combine_mfma_kernel(MfmaArgs a) {
     const int D = kNarrow ? a.d.head_dim : 64 * C;
@@ -1094,14 +1098,15 @@ combine_mfma_kernel(MfmaArgs a) {
     // The wave index as a scalar, so that the per-sequence plan entries below are
     // scalar loads.
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-    const int64_t pair = (int64_t)blockIdx.x * 4 + wave;
+    const int64_t pair = kShare ? (int64_t)blockIdx.x : (int64_t)blockIdx.x * 4 + wave;
     if (pair >= (int64_t)a.d.batch * a.d.num_q_heads) return;
     const int b = uniform(floor_div(pair, a.d.num_q_heads));
     const int hq = (int)(pair - (int64_t)b * a.d.num_q_heads);
     const int32_t t0 = a.plan[b], t1 = a.plan[b + 1];
     const int d4 = lane % kLanesPerPiece, po = lane / kLanesPerPiece;
     if (t1 == t0) {
-        if (po == 0 && (!kNarrow || 4 * d4 < D)) store_out4<QT>(a.d, b, hq, 4 * d4, 0.0f, 0.0f, 0.0f, 0.0f);
+        if (po == 0 && (!kNarrow || 4 * d4 < D) && (!kShare || wave == 0))
+            store_out4<QT>(a.d, b, hq, 4 * d4, 0.0f, 0.0f, 0.0f, 0.0f);
         return;
     }
     const int64_t total = a.plan[a.d.batch];
@@ -1125,7 +1130,7 @@ combine_mfma_kernel(MfmaArgs a) {
     float mr = kNegInf, den = 0.0f;
     float4 num = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
 #pragma unroll 4
-    for (int32_t i = po; i < pieces; i += kPiecesPerPass) {
+    for (int32_t i = kShare ? kPiecesPerPass * wave + po : po; i < pieces; i += kPiecesPerPass * (kShare ? 4 : 1)) {
         const int64_t si = state_index(i);
         const float mi = a.part_m[si];
         const float li = a.part_l[si];
@@ -1152,6 +1157,30 @@ combine_mfma_kernel(MfmaArgs a) {
         num.w = num.w * sa + __shfl_xor(num.w, off) * sb;
         den = den * sa + __shfl_xor(den, off) * sb;
         mr = mn;
+    }
+    if constexpr (kShare) {
+        __shared__ float4 share_num[4][kLanesPerPiece];
+        __shared__ float2 share_md[4][kLanesPerPiece];
+        if (po == 0) {
+            share_num[wave][d4] = num;
+            share_md[wave][d4] = make_float2(mr, den);
+        }
+        __syncthreads();                     // the whole workgroup is here: one pair, one path
+        if (wave != 0) return;
+#pragma unroll
+        for (int v = 1; v < 4; ++v) {
+            const float4 x = share_num[v][d4];
+            const float2 md = share_md[v][d4];
+            const float mn = fmaxf(mr, md.x);
+            const float mu = mn == kNegInf ? 0.0f : mn;
+            const float sa = fast_exp2(mr - mu), sb = fast_exp2(md.x - mu);
+            num.x = num.x * sa + x.x * sb;
+            num.y = num.y * sa + x.y * sb;
+            num.z = num.z * sa + x.z * sb;
+            num.w = num.w * sa + x.w * sb;
+            den = den * sa + md.y * sb;
+            mr = mn;
+        }
     }
     if (po == 0 && (!kNarrow || 4 * d4 < D)) {
         const bool ok = den > 0.0f;
@@ -1232,7 +1261,13 @@ hipError_t launch_w(const MfmaArgs& a, int64_t cap, hipStream_t s, int phases) {
     }
     if (!(phases & kPhaseReduce)) return hipSuccess;
     const int64_t pairs = (int64_t)a.d.batch * a.d.num_q_heads;
-    hipLaunchKernelGGL((combine_mfma_kernel<C, QT, kNarrow>), dim3((unsigned)((pairs + 3) / 4)), dim3(256), 0, s, a);
+    if constexpr (kNarrow) {
+        if (pairs < 4 * (int64_t)device_cus()) {
+            hipLaunchKernelGGL((combine_mfma_kernel<C, QT, true, true>), dim3((unsigned)pairs), dim3(256), 0, s, a);
+            return hipGetLastError();
+        }
+    }
+    hipLaunchKernelGGL((combine_mfma_kernel<C, QT, kNarrow, false>), dim3((unsigned)((pairs + 3) / 4)), dim3(256), 0, s, a);
     return hipGetLastError();
 }
 

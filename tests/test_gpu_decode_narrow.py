@@ -113,6 +113,23 @@ def test_narrow_heads_split_over_the_grid():
         assert t.equal(out, decode_attention_wrapper(q, kv))
 
 
+@pytest.mark.parametrize("q_dtype", [t.bfloat16, t.float32])
+@pytest.mark.parametrize("hq,hkv,d,lengths", [
+    (4, 1, 80, [20000]),                                # hundreds of pieces, four waves per q head
+    (8, 2, 112, [0, 9001, 33, 6000]),
+    (16, 16, 96, [1500] + [40] * 62),                   # one pair short of a wave per SIMD of 256 CUs
+    (16, 16, 96, [1500] + [40] * 63),                   # as many: one wave per q head
+    (32, 8, 80, [3000] * 3 + [100] * 40),
+])
+def test_pieces_of_few_and_many_pairs(q_dtype, hq, hkv, d, lengths):
+    q, kv, k, v = batch(lengths, hq, hkv, d, t.float8_e4m3fn, q_dtype)
+    out = decode_attention_wrapper(q, kv)
+    want = reference(q, k, v, lengths)
+    assert float((out.double() - want).norm()) <= TOLERANCE[q_dtype] * float(want.norm())
+    assert all(not out[b].any() for b, n in enumerate(lengths) if n == 0)
+    assert t.equal(out, decode_attention_wrapper(q, kv))
+
+
 def test_infinite_values_stay_in_their_row():
     """An infinite q element gives infinite scores, not NaN from its zero parts."""
     lengths = [40, 40]
