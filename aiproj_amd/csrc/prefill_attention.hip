@@ -1152,8 +1152,16 @@ extern "C" int kvfp8_prefill_attention(const void* q, const void* k, const void*
                          fa_upx * kXcds * (((int64_t)max_seq_len + fa_rows - 1) / fa_rows) < ((int64_t)1 << 31);
     // It masks and compares unscaled scores, which needs scale > 0: with a negative one masked
     // keys would get infinite weight, with 0 NaN. The general kernel scales first.
-    const bool fa_size = head_dim == 64 || head_dim == 80 || head_dim == 96 || head_dim == 112 || head_dim == 128;
-    if ((dtype == KVFP8_BF16 || dtype == KVFP8_F16) && fa_size && fa_fits && scale > 0.0f) {
+    const bool narrow = head_dim == 80 || head_dim == 96 || head_dim == 112;
+    const bool fa_size = head_dim == 64 || head_dim == 128 || narrow;
+    // A few prompts of 33 to 64 tokens of groups of four q heads are one round of the general
+    // kernel's workgroups of 32 rows, and one item of 64 rows each of the wide kernel. Measured
+    // (us, general against wide): one prompt of 64, 4q/1kv, D 112 7.9, 10.0 and D 80 7.6, 8.5; 16
+    // prompts, 32q/8kv, D 80 9.4, 9.9; with 32 prompts the second round starts, 17.4, 10.9. Two q
+    // heads or fewer per workgroup: 6q/3kv, D 112 7.5, 6.9. 32 tokens: 4q/1kv, D 112 7.7, 7.3.
+    const bool one_round = narrow && a.heads_per_block == 4 && max_seq_len > 32 && max_seq_len <= 64 &&
+                           2 * fa_units <= device_cus();
+    if ((dtype == KVFP8_BF16 || dtype == KVFP8_F16) && fa_size && fa_fits && scale > 0.0f && !one_round) {
         a.rows = fa_rows;
         a.qblocks = (max_seq_len + a.rows - 1) / a.rows;
         // One persistent workgroup per CU (its LDS holds one), per_xcd of them on

@@ -72,3 +72,22 @@ def test_largest_probability_is_exact(dtype, half_ulp, head_dim):
     out, _ = flash_attention_forward(q, k, v, cu, 65, 1 / math.sqrt(head_dim))
     e = t.exp(q[last].double().sum(-1, keepdim=True) / math.sqrt(head_dim))
     t.testing.assert_close(out[last].double(), v[last].double() * (e / (64 + e)), rtol=half_ulp + 4e-6, atol=0)
+
+
+@t.inference_mode()
+@pytest.mark.parametrize("dtype,head_dim", [(t.float16, 80), (t.bfloat16, 112)])
+@pytest.mark.parametrize("count,longest", [(1, 32), (1, 33), (1, 64), (1, 65), (64, 64), (65, 64)])
+def test_short_prompts_around_the_two_kernels(dtype, head_dim, count, longest):
+    """Groups of four q heads: few prompts of 33 to 64 tokens run on the general kernel, up to a workgroup
+    of 32 rows per CU (two KV heads, 64 prompts on 256 CUs); others on the wide one."""
+    lengths = [longest] + [1 + (i * 7) % longest for i in range(1, count)]
+    gen = t.Generator(device="cuda").manual_seed(head_dim)
+    q, k, v = (t.randn(sum(lengths), h, head_dim, device="cuda", generator=gen).to(dtype) for h in (8, 2, 2))
+    cu = t.tensor([0] + list(np.cumsum(lengths)), dtype=t.int32, device="cuda")
+    scale = 1 / math.sqrt(head_dim)
+    out, lse = flash_attention_forward(q, k, v, cu, longest, scale)
+    want, want_lse = oracle.causal_varlen_attention(*(x.double().cpu().numpy() for x in (q, k, v)), cu.cpu().numpy(),
+                                                    longest, scale)
+    tol = TOLERANCE[dtype]
+    t.testing.assert_close(out.double().cpu(), t.from_numpy(want), rtol=tol, atol=tol)
+    t.testing.assert_close(lse.double().cpu(), t.from_numpy(want_lse), rtol=1e-3, atol=1e-3)
