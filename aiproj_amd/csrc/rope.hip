@@ -60,6 +60,10 @@ rope_kernel(RopeArgs a) {
 // attention needs no copies. Bound: HBM, rows read and written once.
 // Measured (4224 rows of 16q/4kv heads, D 128, bf16): one pair per thread with 64-bit index
 // divisions 30 us in place, and 20 us more for the three copies -> 19 us split.
+// In place, few rows are launch and latency: one pair per thread then ends sooner. Measured (us,
+// bf16, one pair | eight elements): 20 heads of 128, 65 rows 2.3 | 2.8, 128 rows (164 thousand
+// pairs) 2.6 | 2.9, 256 rows 3.3 | 3.2; 40 heads of 80, 128 rows (205 thousand) 3.0 | 2.9.
+constexpr int64_t kRopeVecPairs = 200000;
 struct RopeOut {
     void* q;
     void* k;
@@ -195,7 +199,7 @@ extern "C" int kvfp8_rope_inplace(void* x, int dtype, int64_t rows, int32_t head
     if (!x || !positions || !cos_table || !sin_table) return KVFP8_ENULL;
     RopeArgs a{x, rows, heads, head_dim, row_stride, head_stride, positions, pos_dtype == KVFP8_I64,
                cos_table, sin_table, table_rows};
-    if (rope_vec_ok(a, dtype, table_dtype, heads))
+    if (rows * heads * (head_dim / 2) >= kRopeVecPairs && rope_vec_ok(a, dtype, table_dtype, heads))
         return (int)launch_rope_vec<false>(a, RopeOut{}, dtype, table_dtype, rows * heads * (head_dim / 8),
                                            reinterpret_cast<hipStream_t>(stream));
     const int64_t total = rows * heads * (head_dim / 2);

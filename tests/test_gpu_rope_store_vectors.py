@@ -33,6 +33,21 @@ def test_split_equals_the_op_sequence(dtype, head_dim, rows):
     assert t.equal(got.view(rows, -1, head_dim), want)
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("head_dim,heads", [(8, 10), (24, 5), (64, 20), (128, 3)])
+def test_in_place_on_both_sides_of_the_kernels(dtype, head_dim, heads):
+    """The last row count of the pair kernel and the first of the eight-element one (200000 pairs)."""
+    first = -(-200000 // (heads * head_dim // 2))
+    gen = t.Generator(device="cuda").manual_seed(head_dim)
+    rope = RoPE(head_dim, 256, 10000.0).cuda()
+    for rows in (first - 1, first):
+        x = t.randn(rows, heads * head_dim + 16, generator=gen, device="cuda").to(dtype)
+        pos = t.randint(0, 256, (rows,), generator=gen, device="cuda")
+        want = x.clone()
+        want[:, :-16] = rope(x[:, :-16].reshape(rows, heads, head_dim), pos).flatten(1)
+        assert t.equal(rope.apply_(x, pos, heads), want)
+
+
 def test_rows_off_a_16_byte_boundary():
     flat = t.randn(1 + 5 * 4 * 16, device="cuda").to(t.bfloat16)
     x = flat[1:].view(5, 64)
