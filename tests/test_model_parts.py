@@ -123,3 +123,19 @@ def test_an_assigned_bias_is_added(mode, monkeypatch):
     monkeypatch.setattr(RoPE, "apply_", Doubling.apply_)
     q, _ = attend(attn, mode, monkeypatch, x)
     t.testing.assert_close(q.flatten(1), 2 * (x @ attn.qkv_proj.weight.T + attn.qkv_proj.bias)[:, :32])
+
+
+@t.no_grad()
+def test_more_rows_than_the_kernel_takes_cost_no_checks(monkeypatch):
+    """Above 64 rows a projection is torch's GEMM at once: the checks in front of the kernel would be host
+    time of every layer."""
+    def called(x, w):
+        raise AssertionError("checked")
+
+    monkeypatch.setattr(transformer, "_takes_skinny", called)
+    monkeypatch.setattr(transformer, "silu_mul", lambda gu, n: gu[:, :n])
+    monkeypatch.setattr(RoPE, "apply_", Doubling.apply_)
+    h = t.randn(65, CFG.d_model)
+    q, _ = attend(Attention(CFG), "decode", monkeypatch, h)
+    assert q.shape == (65, CFG.num_q_heads, CFG.head_dim)
+    assert SwiGLU(CFG)(h).shape == h.shape
