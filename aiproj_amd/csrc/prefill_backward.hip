@@ -84,8 +84,9 @@ struct BwdArgs {
 // x as three bf16 values, hi + mid + lo = x exactly (normal x); the parts of two floats share
 // a dword. Truncated (kNearest false): the parts have x's sign and reach 2^-7 and 2^-15 of it,
 // for one-plane inputs, where every product is added up. To nearest: 2^-8 and 2^-17, of either
-// sign, for inputs of several planes, where some products are left out. Infinite x leaves NaN
-// parts: non-finite either way.
+// sign, for inputs of several planes, where some products are left out. Infinite x has itself
+// as its first part and NaN as the others: gradients it enters are not finite in any form, and
+// scores are read off the first parts.
 template <bool kNearest>
 __device__ __forceinline__ void split3(float x0, float x1, u32x4_t (&out)[3], int dword) {
     float r0 = x0, r1 = x1;
@@ -301,9 +302,10 @@ __device__ __forceinline__ void bwd_item(const BwdArgs& a, int64_t item, uint8_t
 
     // One sub-block of 32 streamed rows, row0 .. row0 + 31, in rows 32 pp of the buffer.
     auto sub_block = [&](int pp, int row0, uint32_t buf_off, uint32_t stat) __attribute__((always_inline)) {
-        // dP - delta starts from -delta. [1]: the products of lower planes (float32 inputs).
-        constexpr int SUMS = NP == 3 ? 2 : 1;
-        f32x4_t sc[SUMS][2], dp[SUMS][2], lse4[2];
+        // dP - delta starts from -delta. [1]: the products of lower planes, for the scores of
+        // several planes (see below) and dP of float32 inputs.
+        constexpr int SC = NP > 1 ? 2 : 1, DP = NP == 3 ? 2 : 1;
+        f32x4_t sc[SC][2], dp[DP][2], lse4[2];
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             if constexpr (kDq) {
@@ -313,7 +315,8 @@ __device__ __forceinline__ void bwd_item(const BwdArgs& a, int64_t item, uint8_t
                 lse4[h] = *(lds_f32x4*)at;
                 dp[0][h] = -*(lds_f32x4*)(at + 256);
             }
-            if constexpr (SUMS == 2) sc[1][h] = dp[1][h] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+            if constexpr (SC == 2) sc[1][h] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+            if constexpr (DP == 2) dp[1][h] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
         }
 #pragma unroll
         for (int h = 0; h < 2; ++h)
@@ -325,20 +328,24 @@ __device__ __forceinline__ void bwd_item(const BwdArgs& a, int64_t item, uint8_t
                     const u32x4_t x1 = *(lds_u32x4*)at, x2 = *(lds_u32x4*)(at + NP * TB);
 #pragma unroll
                     for (int pb = 0; pb < NP && pa + pb < 3; ++pb) {
-                        const int x = pa + pb > 0 ? SUMS - 1 : 0;
+                        const int x = pa + pb > 0 ? SC - 1 : 0, y = pa + pb > 0 ? DP - 1 : 0;
                         const f32x4_t zero = {0.0f, 0.0f, 0.0f, 0.0f};
                         sc[x][h] = mma16<false>(x1, own1[s][pb], s == 0 && pa + pb == 0 ? zero : sc[x][h]);
-                        dp[x][h] = mma16<false>(x2, own2[s][pb], dp[x][h]);
+                        dp[y][h] = mma16<false>(x2, own2[s][pb], dp[y][h]);
                     }
                 }
         const bool full = kDq ? row0 + 31 <= own0 : (row0 >= own0 + OW - 1 && row0 + 32 <= L);   // wave-uniform
         float pr[2][4];
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-            if constexpr (SUMS == 2) {
-                sc[0][h] += sc[1][h];
-                dp[0][h] += dp[1][h];
+            if constexpr (SC == 2) {
+                // An infinite q or k has NaN in its lower planes, but its score is that of the first
+                // planes: -inf is a weight of zero.
+#pragma unroll
+                for (int jj = 0; jj < 4; ++jj)
+                    sc[0][h][jj] = __builtin_isinf(sc[0][h][jj]) ? sc[0][h][jj] : sc[0][h][jj] + sc[1][h][jj];
             }
+            if constexpr (DP == 2) dp[0][h] += dp[1][h];
 #pragma unroll
             for (int jj = 0; jj < 4; ++jj) {
                 const float lse = kDq ? own_lse : lse4[h][jj];

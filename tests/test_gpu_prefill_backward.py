@@ -185,3 +185,22 @@ def test_every_split_of_four_q_heads(dtype, count, splits):
     check(got, reference(q, k, v, bounds, longest, grad), dtype)
     again = fa._native_backward(q, k, v, out, lse, cu, grad, longest, 0.125)
     assert all(t.equal(a, b) for a, b in zip(got, again))
+
+
+@pytest.mark.parametrize("d", [64, 80, 128, 17])
+@pytest.mark.parametrize("dtype", [t.bfloat16, t.float16])
+@pytest.mark.parametrize("which", [0, 1])
+@pytest.mark.parametrize("value", [math.inf, -math.inf])
+def test_an_infinite_q_or_k_spreads_no_further_than_in_torch(d, dtype, which, value):
+    """A score of -inf is a weight of zero: the rows that PyTorch's operations give finite gradients get
+    the same ones here."""
+    bounds, (q, k, v, grad) = inputs([90, 200, 33], 6, 2, d, dtype, seed=d)
+    (q, k)[which][150, 1, d // 2] = value
+    cu = t.tensor(bounds, dtype=t.int32, device="cuda")
+    out, lse = fa.flash_attention_forward(q, k, v, cu, 200, d ** -0.5)
+    got = fa._native_backward(q, k, v, out, lse, cu, grad, 200, d ** -0.5)
+    strided = grad.transpose(0, 1).contiguous().transpose(0, 1)
+    for g, w in zip(got, fa.flash_attention_backward(q, k, v, out, lse, cu, strided, 200, d ** -0.5)):
+        finite = t.isfinite(w)
+        assert bool(finite.any()) and bool(t.isfinite(g[finite]).all())
+        assert float((g[finite].double() - w[finite].double()).norm()) <= TOLERANCE[dtype] * float(w[finite].double().norm())
