@@ -438,9 +438,10 @@ prefill_attention_kernel(PrefillArgs a) {
 // maximum. Behind it by up to 2^8, as for 64 and 128, the largest probability is rounded to
 // 16 bits while the denominator is not: error against 64 bits 2.47e-4 -> 2.53e-4 for flat
 // rows and 2.16e-4 -> 2.54e-4 for peaked ones (f16, D 80).
-// Measured, 16 prompts of 64 to 1984 tokens, 32q/8kv heads, D 80, f16: 1127 us on the
-// general kernel above (which pads every product to 128 dims) -> 443 us; in another order of
-// the lengths 483 us, and 440 us with the reference of 64 and 128.
+// Measured, 16 prompts of 64 to 1984 tokens, 32q/8kv heads, D 80, f16, in two orders of the
+// lengths: 1031 and 1120 us on the general kernel above (which pads every product to 128
+// dims) -> 438 and 418 us (386 and 367 with the exponents of 64 and 128: the reference behind by
+// up to 2^8 and the scale fused into the subtraction, 3.6% of it the latter).
 //
 // An item is one (sequence, KV head, query block): the eight waves are `gw` q heads
 // x (8 / gw) groups of 32 query rows, and its K/V blocks of 64 keys are staged once
@@ -527,6 +528,12 @@ __device__ __forceinline__ f32x4_t mma16_half(uint2 a, uint2 b, f32x4_t c) {
                                                          0, 0);
 }
 
+// x c + y with the product rounded: 0 where y is the negated rounded product, whatever its size.
+__device__ __forceinline__ float scaled_minus(float x, float c, float y) {
+#pragma clang fp contract(off)
+    return x * c + y;
+}
+
 template <int kD, bool kF16>
 __global__ void __launch_bounds__(kFaThreads)
 prefill_fa_kernel(PrefillArgs a, int32_t units, int32_t upx, int32_t per_xcd) {
@@ -540,7 +547,9 @@ prefill_fa_kernel(PrefillArgs a, int32_t units, int32_t upx, int32_t per_xcd) {
     constexpr bool kHalf = kD % 32 != 0;             // and one step of 16 dims
     // How far (log2) a row's max may exceed the reference that its probabilities are scaled by.
     // 80, 96 and 112: not at all, so that the largest probability is 1 and packed without error,
-    // as on the general kernel (see above).
+    // as on the general kernel (see above). Their scaled scores are rounded before the reference is
+    // taken off for the same reason: a fused product would leave the reference's rounding in the
+    // exponent, which from scores of some 2^30 on is more than the exponent's range.
     constexpr float kLag = kD == 64 || kD == 128 ? 8.0f : 0.0f;
     // Vector-memory instructions a wave issues: kBlockLoads per K/V block, kQLoads
     // for its Q operands of one item.
@@ -840,7 +849,9 @@ prefill_fa_kernel(PrefillArgs a, int32_t units, int32_t upx, int32_t per_xcd) {
         }
         float pr[kFaTiles][16];
         auto prob = [&](int qt, int i) __attribute__((always_inline)) {
-            pr[qt][i] = __builtin_amdgcn_exp2f(__builtin_fmaf(sacc[i / 4][qt][i % 4], a.scale_log2, neg_m[qt]));
+            const float x = sacc[i / 4][qt][i % 4];
+            pr[qt][i] = __builtin_amdgcn_exp2f(kLag > 0.0f ? __builtin_fmaf(x, a.scale_log2, neg_m[qt])
+                                                           : scaled_minus(x, a.scale_log2, neg_m[qt]));
             l[qt] += pr[qt][i];
         };
         auto pack_half = [&](int pp) __attribute__((always_inline)) {

@@ -91,3 +91,28 @@ def test_short_prompts_around_the_two_kernels(dtype, head_dim, count, longest):
     tol = TOLERANCE[dtype]
     t.testing.assert_close(out.double().cpu(), t.from_numpy(want), rtol=tol, atol=tol)
     t.testing.assert_close(lse.double().cpu(), t.from_numpy(want_lse), rtol=1e-3, atol=1e-3)
+
+
+@t.inference_mode()
+@pytest.mark.parametrize("head_dim", [80, 96, 112])
+@pytest.mark.parametrize("size", [1e4, 1e12, 1e30])
+def test_scores_of_any_size(head_dim, size):
+    """One element of q that decides every score: finite, and the value of the key with the largest
+    score, whose weight is 1 (the next one is more than e^100 below)."""
+    gen = t.Generator(device="cuda").manual_seed(head_dim)
+    n = 300
+    q, k, v = (t.randn(n, h, head_dim, device="cuda", generator=gen).to(t.bfloat16) for h in (8, 2, 2))
+    q[:, :, 3] = size
+    k[:, :, 3] = (1 + t.randperm(n, device="cuda", generator=gen) % 64)[:, None] / 16
+    cu = t.tensor([0, n], dtype=t.int32, device="cuda")
+    out, lse = flash_attention_forward(q, k, v, cu, n, 1 / math.sqrt(head_dim))
+    assert bool(t.isfinite(out).all()) and bool(t.isfinite(lse).all())
+    for row in (0, 1, 63, 64, 150, 299):
+        kk = k[:row + 1, 0, 3].float()
+        best = kk == kk.max()
+        if size == 1e4 and int(best.sum()) > 1:
+            continue                                   # there the other dims decide between equal keys
+        want = v[:row + 1, 0].double()[best]
+        low, high = want.amin(0) - 0.02, want.amax(0) + 0.02
+        for h in range(4):
+            assert bool(((out[row, h] >= low) & (out[row, h] <= high)).all())
