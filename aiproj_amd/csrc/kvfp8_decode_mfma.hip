@@ -143,7 +143,8 @@ __device__ __forceinline__ float row_ror8(float x) {
 // past it load the row's last ones again and their q operands are zero. These sizes keep the
 // precision of the vector-ALU kernels they would otherwise take: q and the probabilities
 // enter the products as bf16 parts that hold all of their bits, at most three. (bf16 and
-// f16 caches stay there: an infinite element would multiply parts that are zero.)
+// f16 caches stay there: an infinite element would multiply parts that are zero. Parts below
+// the smallest normal number are lost: V of some 1e-34 keeps 14 bits, of 1e-36 7.)
 // Measured, B 32, 512 to 4096 tokens, 32q/8kv heads, D 80, f16 q, append and decode: 66 us on
 // the vector ALU -> 41 us.
 //

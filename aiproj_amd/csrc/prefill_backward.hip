@@ -81,8 +81,8 @@ struct BwdArgs {
     float* part;                   // their sums [dK, dV][split][T][Hkv][d] when splits > 1
 };
 
-// x as three bf16 values, hi + mid + lo = x exactly (normal x); the parts of two floats share
-// a dword. Truncated (kNearest false): the parts have x's sign and reach 2^-7 and 2^-15 of it,
+// x as three bf16 values, hi + mid + lo = x exactly (|x| above some 1e-33, so that every part is
+// a normal number); the parts of two floats share a dword. Truncated (kNearest false): the parts have x's sign and reach 2^-7 and 2^-15 of it,
 // for one-plane inputs, where every product is added up. To nearest: 2^-8 and 2^-17, of either
 // sign, for inputs of several planes, where some products are left out. Infinite x has itself
 // as its first part and NaN as the others: gradients it enters are not finite in any form, and
