@@ -1086,10 +1086,12 @@ __device__ __forceinline__ int32_t group_of(int64_t x, int64_t total, int64_t gr
 // one piece per lane, acc as float4 runs with D/4 lanes per piece), so the merge
 // costs a couple of memory latencies for the pieces of an ordinary batch.
 // Narrow rows take the lanes of 128 dims per piece; those past the row only follow.
-// kShare (narrow rows, fewer pairs than the chip has SIMDs): the four waves of a workgroup
+// kShare (narrow rows, fewer pairs than the chip has SIMDs, tables of more than kShareTiles tiles,
+// 1024 tokens: a sequence of 2000 gains a fifth, of 500 nothing): the four waves of a workgroup
 // share a pair's pieces, of which a lone long sequence has hundreds. One sequence of 20000
 // tokens, D 80, decode and combine, 4q/1kv and 8q/2kv heads: 51 and 47 us with a wave per pair
 // (37 and 38 on the vector ALU) -> 21 us; 1 to 16 sequences of 500: 9 to 14 us both.
+constexpr int64_t kShareTiles = 64;
 template <int C, int QT, bool kNarrow, bool kShare>
 __global__ void __launch_bounds__(256)
 combine_mfma_kernel(MfmaArgs a) {
@@ -1263,7 +1265,8 @@ hipError_t launch_w(const MfmaArgs& a, int64_t cap, hipStream_t s, int phases) {
     if (!(phases & kPhaseReduce)) return hipSuccess;
     const int64_t pairs = (int64_t)a.d.batch * a.d.num_q_heads;
     if constexpr (kNarrow) {
-        if (pairs < 4 * (int64_t)device_cus()) {
+        const int64_t seq_tiles = a.d.bt_width * (a.d.block_size / 16);
+        if (pairs < 4 * (int64_t)device_cus() && seq_tiles > kShareTiles) {
             hipLaunchKernelGGL((combine_mfma_kernel<C, QT, true, true>), dim3((unsigned)pairs), dim3(256), 0, s, a);
             return hipGetLastError();
         }

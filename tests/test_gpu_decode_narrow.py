@@ -117,6 +117,8 @@ def test_narrow_heads_split_over_the_grid():
 @pytest.mark.parametrize("hq,hkv,d,lengths", [
     (4, 1, 80, [20000]),                                # hundreds of pieces, four waves per q head
     (8, 2, 112, [0, 9001, 33, 6000]),
+    (8, 1, 80, [1008, 700]),                            # tables of 64 pages: one wave per q head
+    (8, 1, 80, [1009, 700]),                            # of 65: four
     (16, 16, 96, [1500] + [40] * 62),                   # one pair short of a wave per SIMD of 256 CUs
     (16, 16, 96, [1500] + [40] * 63),                   # as many: one wave per q head
     (32, 8, 80, [3000] * 3 + [100] * 40),
